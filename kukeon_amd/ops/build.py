@@ -126,6 +126,7 @@ SOURCES = [
     "activation.hip",
     "rope_kv.hip",
     "paged_attn.hip",
+    "prompt_attn.hip",
     "prefill_attn.hip",
     "sampling.hip",
     "moe.hip",

@@ -1,10 +1,10 @@
-// Varlen causal paged prefill attention (MFMA, bf16) for gfx950, also in a
-// chunk-local form with capped scores (template flag EXT) — plus the
-// fragment-layout probe used by the GPU test suite to pin the
-// v_mfma_f32_32x32x16_bf16 operand maps this kernel relies on.
+// Varlen paged prompt attention (MFMA, bf16) for gfx950 in the forms of the
+// hybrid stacks: chunk-local, windowed, capped scores, distance biases, sinks
+// (prompt_attn.hip has the plain causal one) — plus the fragment-layout probe
+// used by the GPU test suite to pin the v_mfma_f32_32x32x16_bf16 operand maps
+// that these kernels rely on.
 //
-// Structure (MI355X-first; guide §Appendix B attention recipe adapted to a
-// paged varlen serving kernel):
+// Structure:
 //   - workgroup = 4 waves = the 4 q-heads of one GQA group (K/V staged in
 //     LDS once per 32-token tile and shared by all heads: KV HBM traffic is
 //     never multiplied by the group size); grid.z splits groups of 8.
@@ -123,10 +123,10 @@ DEV_INLINE unsigned int cvt_pk_bf16(float lo, float hi) {
 
 // ---------- the kernel ----------
 // D=128, QBLK=32 rows per workgroup, KV tile = 32 tokens (2 cache blocks).
-// EXT adds what chunk-local attention with capped scores needs: keys start at
+// For chunk-local attention with capped scores, keys start at
 // the first position of the query's chunk, scores pass cap * tanh(s / cap),
 // and the softmax weights enter the PV product as hi + lo (two bf16 terms)
-// so that they keep fp32-grade accuracy. EXT also serves a sliding window
+// so that they keep fp32-grade accuracy. EXT == 1 also serves a sliding window
 // (keys from q - window + 1 on, and positions below `keep`, whose tiles come
 // ahead of the window's), a distance bias slope_h (q - k) taken off head h's
 // scores, and a sink per head: the softmax starts from a score that has no
@@ -135,11 +135,11 @@ DEV_INLINE unsigned int cvt_pk_bf16(float lo, float hi) {
 // r1_h ln(1 + r2_h (q - k)) (a wave's 63 distances of a tile are one logarithm
 // per lane, handed over through LDS) and keys divided by their own root mean
 // square (formed while the tile is staged).
-template <int BS, bool FP8, int EXT>
+template <int BS, int EXT>
 __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
     unsigned short* __restrict__ out,       // [T, Hq*D]
     const unsigned short* __restrict__ q,   // [T, q_stride] fused qkv rows
-    const void* __restrict__ k_cache,       // [NB, Hk, BS, D] bf16|fp8
+    const void* __restrict__ k_cache,       // [NB, Hk, BS, D] bf16
     const void* __restrict__ v_cache,
     const int* __restrict__ block_table,    // [nseq, max_blocks]
     const int* __restrict__ seq_lens,       // [nseq] total ctx after append
@@ -180,13 +180,13 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
   // absolute position of this lane's q column (clamped for padding rows)
   const int q_abs = abs_start + qb0 + min(qcol, qn - 1);
   // first key this lane's query sees, and the first any row of the tile sees
-  int q_lo = (EXT && chunk > 0) ? (q_abs / chunk) * chunk : 0;
-  int tile_lo = (EXT && chunk > 0) ? ((abs_start + qb0) / chunk) * chunk : 0;
-  if (EXT && window > 0) {
+  int q_lo = chunk > 0 ? (q_abs / chunk) * chunk : 0;
+  int tile_lo = chunk > 0 ? ((abs_start + qb0) / chunk) * chunk : 0;
+  if (window > 0) {
     q_lo = max(q_lo, q_abs - window + 1);
     tile_lo = max(tile_lo, abs_start + qb0 - window + 1);
   }
-  const float slope = (EXT && slopes) ? slopes[head] : 0.f;
+  const float slope = slopes ? slopes[head] : 0.f;
   const float lb1 = (EXT == 2 && r1) ? r1[head] : 0.f;
   const float lb2 = (EXT == 2 && r1) ? r2[head] : 0.f;
 
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
   }
 
   float m = -INFINITY, l_acc = 0.f;
-  if (EXT && sinks) { m = sinks[head]; l_acc = 1.f; }
+  if (sinks) { m = sinks[head]; l_acc = 1.f; }
   f32x16_t oacc[4] = {{}, {}, {}, {}};
 
   const int kv_limit = min(ctx, abs_start + qb0 + qn);
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
 
   // tiles of kept first tokens, then the ones from the first visible key on
   const int tfirst = tile_lo / KVT;
-  const int nkept = EXT ? min(tfirst, (keep + KVT - 1) / KVT) : 0;
+  const int nkept = min(tfirst, (keep + KVT - 1) / KVT);
   for (int it = 0; it < nkept + ntiles - tfirst; ++it) {
     const int ti = it < nkept ? it : tfirst + it - nkept;
     const int kvbase = ti * KVT;
@@ -231,16 +231,9 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
       float kk = 0.f;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        uint4 v;
-        if (FP8) {
-          v = fp8x8_to_bf16x8(*reinterpret_cast<const uint2*>(
-              reinterpret_cast<const unsigned char*>(k_cache) + koff + d0 +
-              c * 8));
-        } else {
-          v = *reinterpret_cast<const uint4*>(
-              reinterpret_cast<const unsigned short*>(k_cache) + koff + d0 +
-              c * 8);
-        }
+        const uint4 v = *reinterpret_cast<const uint4*>(
+            reinterpret_cast<const unsigned short*>(k_cache) + koff + d0 +
+            c * 8);
         const int byte = tok * 256 + (((d0 + c * 8) * 2) ^ swz);
         *reinterpret_cast<uint4*>(
             reinterpret_cast<char*>(kbuf) + byte) = v;
@@ -273,20 +266,10 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
       const long voff1 =
           (((long)block_table[(long)s * max_blocks + vb1] * Hk + hk) * BS +
            (vpos1 % BS)) * D;
-      uint4 r0, r1;
-      if (FP8) {
-        const unsigned char* v8 =
-            reinterpret_cast<const unsigned char*>(v_cache);
-        r0 = fp8x8_to_bf16x8(
-            *reinterpret_cast<const uint2*>(v8 + voff0 + vd0));
-        r1 = fp8x8_to_bf16x8(
-            *reinterpret_cast<const uint2*>(v8 + voff1 + vd0));
-      } else {
-        const unsigned short* v16 =
-            reinterpret_cast<const unsigned short*>(v_cache);
-        r0 = *reinterpret_cast<const uint4*>(v16 + voff0 + vd0);
-        r1 = *reinterpret_cast<const uint4*>(v16 + voff1 + vd0);
-      }
+      const unsigned short* v16 =
+          reinterpret_cast<const unsigned short*>(v_cache);
+      uint4 r0 = *reinterpret_cast<const uint4*>(v16 + voff0 + vd0);
+      uint4 r1 = *reinterpret_cast<const uint4*>(v16 + voff1 + vd0);
       // zero V rows past ctx: a 0*NaN in the PV mfma would poison O
       if (vpos0 >= ctx) r0 = uint4{0, 0, 0, 0};
       if (vpos1 >= ctx) r1 = uint4{0, 0, 0, 0};
@@ -335,7 +318,7 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
       const int kvrow = (r & 3) + 8 * (r >> 2) + 4 * hi;
       const int kvpos = kvbase + kvrow;
       const bool valid = (kvpos <= q_abs) && (kvpos < ctx) &&
-                         (!EXT || kvpos >= q_lo || kvpos < keep);
+                         (kvpos >= q_lo || kvpos < keep);
       float sc;
       if (EXT == 2) {
         sc = sacc[r] * kscale[kvrow];
@@ -346,8 +329,8 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
         sc -= dbias[wid][qcol - kvrow + 31];
       } else {
         sc = sacc[r] * scale;
-        if (EXT && cap > 0.f) sc = cap * tanhf(sc / cap);
-        if (EXT) sc -= slope * (float)(q_abs - kvpos);
+        if (cap > 0.f) sc = cap * tanhf(sc / cap);
+        sc -= slope * (float)(q_abs - kvpos);
       }
       sv[r] = valid ? sc : -INFINITY;
       tmax = fmaxf(tmax, sv[r]);
@@ -387,7 +370,7 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
     }
     // what the rounding to bf16 dropped, as a second set of fragments
     unsigned int pl[2][4];
-    if (EXT) {
+    {
       unsigned int cl[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -420,11 +403,10 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
             as_frag(vf.x, vf.y, vf.z, vf.w),
             as_frag(pb[c][0], pb[c][1], pb[c][2], pb[c][3]),
             oacc[db], 0, 0, 0);
-        if (EXT)
-          oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              as_frag(vf.x, vf.y, vf.z, vf.w),
-              as_frag(pl[c][0], pl[c][1], pl[c][2], pl[c][3]),
-              oacc[db], 0, 0, 0);
+        oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            as_frag(vf.x, vf.y, vf.z, vf.w),
+            as_frag(pl[c][0], pl[c][1], pl[c][2], pl[c][3]),
+            oacc[db], 0, 0, 0);
       }
     }
   }
@@ -446,39 +428,6 @@ __global__ __launch_bounds__(256, EXT == 2 ? 2 : 1) void prefill_attn_kernel(
       *reinterpret_cast<uint2*>(orow + d) = uint2{w0, w1};
     }
   }
-}
-
-void prefill_attention(torch::Tensor out, torch::Tensor q,
-                       torch::Tensor k_cache, torch::Tensor v_cache,
-                       torch::Tensor block_table, torch::Tensor seq_lens,
-                       torch::Tensor q_starts, torch::Tensor qb_seq,
-                       torch::Tensor qb_start, int64_t q_offset, double scale) {
-  const int Hk = k_cache.size(1);
-  const int BS = k_cache.size(2);
-  const int D = k_cache.size(3);
-  const int Hq = out.size(1) / D;
-  const int G = Hq / Hk;
-  const int nqb = qb_seq.size(0);
-  if (nqb == 0) return;
-  TORCH_CHECK(D == 128, "only head_dim=128 supported");
-  TORCH_CHECK(BS == 16, "kv block size must be 16");
-  TORCH_CHECK(q_starts.dim() == 2 && q_starts.size(1) == 2);
-  TORCH_CHECK(qb_seq.scalar_type() == torch::kInt32);
-  auto stream = c10::hip::getCurrentHIPStream().stream();
-  dim3 grid(nqb, Hk, (G + 3) / 4);
-  const bool fp8 = k_cache.scalar_type() == torch::kUInt8;
-#define PF_LAUNCH(FP8_)                                                      \
-  prefill_attn_kernel<16, FP8_, 0><<<grid, 256, 0, stream>>>(            \
-      reinterpret_cast<unsigned short*>(out.data_ptr()),                     \
-      reinterpret_cast<const unsigned short*>(q.data_ptr()),                 \
-      k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr<int>(),   \
-      seq_lens.data_ptr<int>(), q_starts.data_ptr<int>(),                    \
-      qb_seq.data_ptr<int>(), qb_start.data_ptr<int>(), q.stride(0),         \
-      q_offset, Hq, Hk, (int)block_table.size(1), (int)out.stride(0),        \
-      (float)scale, 0.f, 0, 0, nullptr, nullptr, nullptr, -1.f, nullptr, 0)
-  if (fp8) { PF_LAUNCH(true); } else { PF_LAUNCH(false); }
-#undef PF_LAUNCH
-  HIP_CHECK_KERNEL();
 }
 
 // sizes the tile kernel serves for chunk-local attention
@@ -521,7 +470,7 @@ void chunk_attention_tiles(torch::Tensor out, torch::Tensor q,
   const int G = Hq / Hk;
   auto stream = c10::hip::getCurrentHIPStream().stream();
   dim3 grid(nqb, Hk, (G + 3) / 4);
-  prefill_attn_kernel<16, false, 1><<<grid, 256, 0, stream>>>(
+  prefill_attn_kernel<16, 1><<<grid, 256, 0, stream>>>(
       reinterpret_cast<unsigned short*>(out.data_ptr()),
       reinterpret_cast<const unsigned short*>(q.data_ptr()),
       k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr<int>(),
@@ -575,7 +524,7 @@ void window_attention_tiles(torch::Tensor out, torch::Tensor q,
   const int G = Hq / Hk;
   auto stream = c10::hip::getCurrentHIPStream().stream();
   dim3 grid(nqb, Hk, (G + 3) / 4);
-  prefill_attn_kernel<16, false, 1><<<grid, 256, 0, stream>>>(
+  prefill_attn_kernel<16, 1><<<grid, 256, 0, stream>>>(
       reinterpret_cast<unsigned short*>(out.data_ptr()),
       reinterpret_cast<const unsigned short*>(q.data_ptr()),
       k_cache.data_ptr(), k_cache.data_ptr(), block_table.data_ptr<int>(),
@@ -636,7 +585,7 @@ void masked_attention_tiles(torch::Tensor out, torch::Tensor q,
   auto stream = c10::hip::getCurrentHIPStream().stream();
   dim3 grid(nqb, Hk, (G + 3) / 4);
 #define KK_LAUNCH(EXT_)                                                      \
-  prefill_attn_kernel<16, false, EXT_><<<grid, 256, 0, stream>>>(            \
+  prefill_attn_kernel<16, EXT_><<<grid, 256, 0, stream>>>(            \
       reinterpret_cast<unsigned short*>(out.data_ptr()),                     \
       reinterpret_cast<const unsigned short*>(q.data_ptr()),                 \
       k_cache.data_ptr(), v_cache.data_ptr(), block_table.data_ptr<int>(),   \

@@ -294,6 +294,47 @@ def test_prefill_continuation():
     _prefill_case([(200, 150), (90, 64), (70, 69)], Hq=8, Hk=2)
 
 
+# tile and block edges (64 keys, 32 and 64 rows), blocks that pair up and
+# blocks that do not, key splits (few rows on a long context), head groups
+# that fill a workgroup's four heads and that do not
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hk,seqs", [
+    (8, 2, [(1, 0), (32, 0), (33, 0), (64, 0), (65, 0), (95, 0), (97, 0)]),
+    (4, 2, [(63, 31), (64, 32), (65, 33), (129, 128), (127, 95), (192, 64)]),
+    (5, 1, [(31, 0), (20, 3), (16, 15)]),
+    (8, 1, [(2050, 2017), (1999, 1998)]),
+    (8, 8, [(1217, 1150)]),
+])
+def test_prefill_tiles(Hq, Hk, seqs, fp8):
+    _prefill_case(seqs, Hq=Hq, Hk=Hk, seed=len(seqs), fp8=fp8)
+
+
+def test_prefill_part_of_the_blocks():
+    """Rows of blocks that are not listed stay as they are, whichever of two
+    neighbouring blocks is listed."""
+    torch.manual_seed(4)
+    D, Hq, Hk, n = 128, 4, 1, 200
+    kc, vc = _make_cache(14, Hk, 16, D)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    bt = torch.arange(13, **i32)[None].contiguous()
+    q = torch.randn(n, Hq * D, dtype=torch.bfloat16, device=DEV)
+    sl = torch.tensor([n], **i32)
+    qs = torch.tensor([[0, 0]], **i32)
+    ref = torch.empty(n, Hq * D, dtype=torch.bfloat16)
+    reference.prefill_attention(ref, q.cpu(), kc.cpu(), vc.cpu(), bt.cpu(),
+                                sl.cpu(), qs.cpu(), None, None, 0, D ** -0.5)
+    for starts in ([32], [0], [32, 64], [0, 64, 96], [64, 32], [96, 160]):
+        out = torch.full((n, Hq * D), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.prefill_attention(out, q, kc, vc, bt, sl, qs,
+                              torch.zeros(len(starts), **i32),
+                              torch.tensor(starts, **i32), 0, D ** -0.5)
+        want = torch.full_like(ref, 7.0)
+        for s in starts:
+            want[s: s + 32] = ref[s: s + 32]
+        torch.testing.assert_close(out.cpu().float(), want.float(),
+                                   rtol=2.5e-2, atol=2.5e-2)
+
+
 def test_prefill_gqa8():
     _prefill_case([(77, 0), (130, 40)], Hq=8, Hk=1)
 
