@@ -110,21 +110,7 @@ class LlamaAttention(nn.Module):
 
     def forward(self, x: torch.Tensor, cos_sin: torch.Tensor,
                 kc: torch.Tensor, vc: torch.Tensor, meta: AttnMeta):
-        qkv = ops.linear(x, self.qkv_w)
-        ops.rope_kv_append(qkv, kc, vc, cos_sin, meta.positions,
-                           meta.slot_mapping, self.hq, self.hk, self.d,
-                           block_table=(meta.block_table
-                                        if meta.mode == "decode" else None))
-        out = torch.empty(x.shape[0], self.hq * self.d, dtype=x.dtype,
-                          device=x.device)
-        if meta.mode == "decode":
-            ops.paged_attention(out, qkv, kc, vc, meta.block_table,
-                                meta.seq_lens, 0, meta.num_splits, self.scale,
-                                meta.tmp_out, meta.tmp_ml)
-        else:
-            ops.prefill_attention(out, qkv, kc, vc, meta.block_table,
-                                  meta.seq_lens, meta.q_starts, meta.qb_seq,
-                                  meta.qb_start, 0, self.scale)
+        out = self.forward_pre_o(x, cos_sin, kc, vc, meta)
         o = ops.linear(out, self.o_w)
         return parallel.tp_all_reduce(o)
 
@@ -133,11 +119,12 @@ class LlamaAttention(nn.Module):
         """Attention WITHOUT the output projection: the layer fuses the
         o-proj with the post-attention add+RMSNorm (one epilogue kernel
         instead of reduce + norm)."""
-        qkv = ops.linear(x, self.qkv_w)
-        ops.rope_kv_append(qkv, kc, vc, cos_sin, meta.positions,
-                           meta.slot_mapping, self.hq, self.hk, self.d,
-                           block_table=(meta.block_table
-                                        if meta.mode == "decode" else None))
+        qkv = ops.qkv_rope_append(x, self.qkv_w, kc, vc, cos_sin,
+                                  meta.positions, meta.slot_mapping, self.hq,
+                                  self.hk, self.d,
+                                  block_table=(meta.block_table
+                                               if meta.mode == "decode"
+                                               else None))
         out = torch.empty(x.shape[0], self.hq * self.d, dtype=x.dtype,
                           device=x.device)
         if meta.mode == "decode":
@@ -161,10 +148,7 @@ class LlamaMLP(nn.Module):
         self.down_w = _init_weight((cfg.hidden_size, self.inter), device)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        gu = ops.linear(x, self.gate_up_w)
-        act = torch.empty(x.shape[0], self.inter, dtype=x.dtype,
-                          device=x.device)
-        ops.silu_mul(act, gu)
+        act = ops.mlp_act(x, self.gate_up_w)
         return parallel.tp_all_reduce(ops.linear(act, self.down_w))
 
 
@@ -205,9 +189,8 @@ class LlamaLayer(nn.Module):
         attn_out = self.attn.forward_pre_o(h, cos_sin, kc, vc, meta)
         h2 = ops.linear_add_rmsnorm(attn_out, self.attn.o_w, residual,
                                     self.post_norm, self.eps)
-        gu = ops.linear(h2, self.mlp.gate_up_w)
-        h_next = ops.mlp_down_fused(gu, self.mlp.down_w, residual,
-                                    next_norm_w, eps)
+        h_next = ops.mlp_fused(h2, self.mlp.gate_up_w, self.mlp.down_w,
+                               residual, next_norm_w, eps)
         return h_next, residual
 
     # -- pipelined TP prefill phases (comm/GEMM overlap): the o-proj and
@@ -228,10 +211,7 @@ class LlamaLayer(nn.Module):
     def part_mlp(self, o_reduced, residual):
         ops.fused_add_rmsnorm(o_reduced, residual, self.post_norm, self.eps)
         h = o_reduced
-        gu = ops.linear(h, self.mlp.gate_up_w)
-        act = torch.empty(h.shape[0], self.mlp.inter, dtype=h.dtype,
-                          device=h.device)
-        ops.silu_mul(act, gu)
+        act = ops.mlp_act(h, self.mlp.gate_up_w)
         return ops.linear(act, self.mlp.down_w)
 
 

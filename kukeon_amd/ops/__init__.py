@@ -354,9 +354,52 @@ def _skinny5_wins(rows: int, N: int, K: int) -> bool:
     return N % 2048 == 0 and N <= 8192 and K % 128 == 0 and K >= 3 * N
 
 
+def _stream_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x @ w.T goes to the weight-streaming kernel (stream_gemm.hip):
+    a decode batch of up to 64 plain bf16 rows against a matrix of at least
+    4 MB (2 MB: 5.6 us against hipBLASLt's 5.8), in the kernel's units of 128
+    rows and 256 columns."""
+    return (_C is not None and _USE_SKINNY == "0" and x.is_cuda
+            and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= 64
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and x.shape[1] == w.shape[1] and w.device == x.device
+            and w.shape[0] % 128 == 0 and w.shape[1] % 256 == 0
+            and w.numel() >= 1 << 21
+            and x.is_contiguous() and w.is_contiguous()
+            # what records, batches or traces goes through torch
+            and type(x) is torch.Tensor
+            and type(w) in (torch.Tensor, torch.nn.Parameter)
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad))
+            and not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0
+            and not torch.jit.is_tracing()
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def _stream_wins(rows: int, N: int, K: int) -> bool:
+    """Where the streaming kernel beats hipBLASLt although nothing takes its
+    partial sums (us, this against hipBLASLt, in a graph, weights from HBM):
+    up to 16 rows everywhere (2048 x 2048 8 to 11, 4096 x 1024 7 to 7.5, 6144 x
+    4096 15 to 16, 28672 x 4096 45 to 64); with more rows adding the parts up
+    costs what the stream gains (6144 x 2048 at 32 rows 13.2 to 12.4), unless
+    the reduction is long (4096 x 14336 28 to 34 at 32 rows, 34 to 41 at 64) or
+    there are enough output columns to need no parts, and not so many that
+    hipBLASLt's tiles fill the chip (28672 x 4096 52 to 63 at 48 rows, 32000 x
+    8192 106 to 134, but 128256 x 4096 213 to 207)."""
+    return (rows <= 16 or K >= 3 * N
+            or (rows <= 48 and 24576 <= N <= 32768))
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """F.linear with the weight-streaming skinny-GEMM kernel on the decode
-    shapes where it measured faster than hipBLASLt; hipBLASLt otherwise."""
+    """F.linear with a weight-streaming kernel on the decode shapes where it
+    measured faster than hipBLASLt; hipBLASLt otherwise."""
+    if (_stream_ok(x, w)
+            and _stream_wins(x.shape[0], w.shape[0], w.shape[1])):
+        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
+                          device=x.device)
+        _C.stream_gemm(out, x, w)
+        return out
     rows = x.shape[0]
     if _C is None:
         # the weight-streaming kernels are an optimisation over the vendor
@@ -431,6 +474,11 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor,
     from kukeon_amd import parallel
     rows = x.shape[0]
     N, K = w.shape
+    if (parallel.tp_size() == 1 and N % 2048 == 0 and N <= 8192
+            and residual.is_contiguous() and _stream_ok(x, w)):
+        normed = torch.empty(rows, N, dtype=x.dtype, device=x.device)
+        _C.stream_gemm_norm(normed, x, w, residual, norm_weight, eps)
+        return normed
     if (x.is_cuda and parallel.tp_size() == 1 and x.dim() == 2
             and rows <= 64 and N % 2048 == 0 and N <= 8192 and K % 128 == 0
             and x.dtype == torch.bfloat16
@@ -512,6 +560,54 @@ def mlp_down_fused(gu: torch.Tensor, w: torch.Tensor,
     act = torch.empty(rows, K, dtype=gu.dtype, device=gu.device)
     silu_mul(act, gu)
     return linear_add_rmsnorm(act, w, residual, norm_weight, eps)
+
+
+def mlp_act(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x Wg^T) * (x Wu^T) for the fused projection w = [Wg; Wu]. Decode
+    batches do it in one kernel, with both factors in fp32; otherwise the
+    projection is rounded to bf16 in between."""
+    act = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
+                      device=x.device)
+    if w.shape[0] % 256 == 0 and _stream_ok(x, w):
+        _C.stream_gemm_silu(act, x, w)
+    else:
+        silu_mul(act, linear(x, w))
+    return act
+
+
+def mlp_fused(x: torch.Tensor, gate_up_w: torch.Tensor,
+              down_w: torch.Tensor, residual: torch.Tensor,
+              norm_weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """The whole gated MLP with the residual add and the norm that follows;
+    updates `residual` and returns the normed rows."""
+    if _FUSE_SILU:
+        return mlp_down_fused(linear(x, gate_up_w), down_w, residual,
+                              norm_weight, eps)
+    return linear_add_rmsnorm(mlp_act(x, gate_up_w), down_w, residual,
+                              norm_weight, eps)
+
+
+def qkv_rope_append(x: torch.Tensor, w: torch.Tensor, k_cache, v_cache,
+                    cos_sin, positions, slot_mapping, num_q_heads: int,
+                    num_kv_heads: int, head_dim: int,
+                    block_table=None) -> torch.Tensor:
+    """The fused q/k/v projection of x, rotary positions and the page write.
+    -> [T, (Hq + 2 Hk) D], of which the query columns are meant to be read
+    (decode batches leave the others unwritten: keys and values go from the
+    projection's fp32 sums straight to their page)."""
+    if _stream_ok(x, w) and head_dim % 16 == 0:
+        if block_table is None:
+            block_table = torch.empty(0, dtype=torch.int32, device=x.device)
+        qkv = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
+                          device=x.device)
+        _C.qkv_rope_append(qkv, x, w, k_cache, v_cache, cos_sin, positions,
+                           slot_mapping, num_q_heads, num_kv_heads, head_dim,
+                           block_table)
+        return qkv
+    qkv = linear(x, w)
+    rope_kv_append(qkv, k_cache, v_cache, cos_sin, positions, slot_mapping,
+                   num_q_heads, num_kv_heads, head_dim, block_table)
+    return qkv
 
 
 def moe_router_weights(wdense, logits, k: int) -> None:

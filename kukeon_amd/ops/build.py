@@ -131,6 +131,7 @@ SOURCES = [
     "sampling.hip",
     "moe.hip",
     "skinny_gemm.hip",
+    "stream_gemm.hip",
     "bindings.cpp",
 ]
 

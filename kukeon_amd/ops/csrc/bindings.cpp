@@ -46,6 +46,16 @@ void skinny_gemm5_silu_fused_norm(torch::Tensor normed, torch::Tensor gu,
                                   double eps);
 void skinny_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                  torch::Tensor ws);
+void stream_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w);
+void stream_gemm_silu(torch::Tensor out, torch::Tensor x, torch::Tensor w);
+void stream_gemm_norm(torch::Tensor normed, torch::Tensor x, torch::Tensor w,
+                      torch::Tensor residual, torch::Tensor nw, double eps);
+void qkv_rope_append(torch::Tensor qkv, torch::Tensor x, torch::Tensor w,
+                     torch::Tensor k_cache, torch::Tensor v_cache,
+                     torch::Tensor cos_sin, torch::Tensor positions,
+                     torch::Tensor slot_mapping, int64_t num_q_heads,
+                     int64_t num_kv_heads, int64_t head_dim,
+                     torch::Tensor block_table);
 void glds_probe(torch::Tensor out, torch::Tensor src);
 void skinny_gemm5_fused_norm(torch::Tensor normed, torch::Tensor x,
                              torch::Tensor w, torch::Tensor ws,
@@ -78,6 +88,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "in-place NEOX RoPE on fused qkv + paged KV append");
   m.def("paged_attention", &kukeon::paged_attention,
         "decode paged attention (GQA, split-KV)");
+  m.def("stream_gemm", &kukeon::stream_gemm,
+        "x W^T for up to 64 rows, streaming W (bf16)");
+  m.def("stream_gemm_silu", &kukeon::stream_gemm_silu,
+        "silu(x Wg^T) * (x Wu^T) for up to 64 rows");
+  m.def("stream_gemm_norm", &kukeon::stream_gemm_norm,
+        "residual += x W^T, RMS norm, for up to 64 rows");
+  m.def("qkv_rope_append", &kukeon::qkv_rope_append,
+        "qkv projection, rotary embedding and page write, up to 64 rows");
   m.def("prefill_attention", &kukeon::prefill_attention,
         "varlen causal paged prefill attention (MFMA)");
   m.def("mfma_probe", &kukeon::mfma_probe,

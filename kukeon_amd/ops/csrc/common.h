@@ -59,11 +59,15 @@ DEV_INLINE uint4 pack_bf16x8(const float* f) {
 // ---------- fp8 (OCP e4m3fn) helpers ----------
 typedef __attribute__((__vector_size__(2 * sizeof(float)))) float f32x2_cvt_t;
 
+typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16
+    bf16x2_cvt_t;
+
+// Two floats to bf16, nearest even, in one v_cvt_pk_bf16_f32 (through
+// __float22bfloat162_rn it came out as two of them, a shift and an or).
 DEV_INLINE unsigned int cvtpk_bf16(float lo, float hi) {
-  __hip_bfloat162 h = __float22bfloat162_rn(float2{lo, hi});
-  unsigned int r;
-  __builtin_memcpy(&r, &h, 4);
-  return r;
+  return __builtin_bit_cast(
+      unsigned int,
+      __builtin_convertvector((f32x2_cvt_t){lo, hi}, bf16x2_cvt_t));
 }
 
 // 4 fp8 bytes (one dword) -> 4 bf16 (uint2)

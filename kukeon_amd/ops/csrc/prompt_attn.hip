@@ -61,15 +61,6 @@ constexpr int BS = 16;          // tokens per page
 constexpr int KVT = 64;         // keys per tile
 constexpr float NONE = -3.0e38f;  // running maximum before any key
 
-typedef __attribute__((__vector_size__(2 * sizeof(float)))) float pair_t;
-typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bpair_t;
-
-// one v_cvt_pk_bf16_f32
-DEV_INLINE unsigned int pack2(float lo, float hi) {
-  return __builtin_bit_cast(unsigned int,
-                            __builtin_convertvector(pair_t{lo, hi}, bpair_t));
-}
-
 struct frag_words { unsigned int x[4]; };
 struct frag_pair { frag4_t lo, hi; };
 
@@ -323,7 +314,7 @@ __global__ __launch_bounds__(NW * WAVE, 2) void prompt_attn_kernel(
         const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[kt][r + 1], c2, -mc));
         ls[r & 2] += p0;
         ls[(r & 2) + 1] += p1;
-        pw[kt][r >> 1] = pack2(p0, p1);
+        pw[kt][r >> 1] = cvtpk_bf16(p0, p1);
       }
     l_acc += (ls[0] + ls[1]) + (ls[2] + ls[3]);
   };
@@ -397,8 +388,8 @@ __global__ __launch_bounds__(NW * WAVE, 2) void prompt_attn_kernel(
 #pragma unroll
     for (int qd = 0; qd < 4; ++qd)
       *reinterpret_cast<uint2*>(orow + db * 32 + qd * 8 + 4 * hi) =
-          uint2{pack2(oacc[db][qd * 4] * inv, oacc[db][qd * 4 + 1] * inv),
-                pack2(oacc[db][qd * 4 + 2] * inv,
+          uint2{cvtpk_bf16(oacc[db][qd * 4] * inv, oacc[db][qd * 4 + 1] * inv),
+                cvtpk_bf16(oacc[db][qd * 4 + 2] * inv,
                            oacc[db][qd * 4 + 3] * inv)};
 }
 
@@ -433,7 +424,7 @@ __global__ __launch_bounds__(256) void prompt_attn_merge_kernel(
   }
   const float inv = l != 0.f ? 1.f / l : 0.f;
   *reinterpret_cast<unsigned int*>(out + row * out_stride + (long)head * D +
-                                   d) = pack2(a0 * inv, a1 * inv);
+                                   d) = cvtpk_bf16(a0 * inv, a1 * inv);
 }
 
 }  // namespace

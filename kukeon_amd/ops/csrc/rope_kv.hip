@@ -15,9 +15,17 @@
 
 namespace kukeon {
 
-template <bool FP8>
+torch::Tensor stream_gemm_sums(torch::Tensor x, torch::Tensor w);
+
+// A thread takes 8 pairs of one head (queries, then keys) or 8 entries of a
+// value row; the three kinds are numbered through, so that a decode batch does
+// them side by side. SUMS: the projection arrives as fp32 parts [splits, T,
+// row] that are added up here; queries go to qkv rounded once, keys and values
+// to their pages only.
+template <bool FP8, bool SUMS>
 __global__ void rope_kv_kernel(
     unsigned short* __restrict__ qkv,        // [T, (Hq+2Hk)*D]
+    const float* __restrict__ sums, int splits,
     void* __restrict__ k_cache,              // [NB, Hk, BS, D] bf16|fp8
     void* __restrict__ v_cache,
     const float* __restrict__ cos_sin,       // [max_pos, D]
@@ -44,89 +52,82 @@ __global__ void rope_kv_kernel(
     slot = slot_mapping[t];
   }
   const float* cs = cos_sin + (long)pos * D;
-
-  // ---- rotate q (in place) ----
-  const int q_chunks = Hq * (D / 16);  // 8 pairs per chunk
-  for (int c = yoff; c < q_chunks; c += ystride) {
-    const int h = c / (D / 16);
-    const int d0 = (c % (D / 16)) * 8;
-    unsigned short* base = row + (long)h * D;
-    bf16x8 x = load_bf16x8(base + d0);
-    bf16x8 y = load_bf16x8(base + half + d0);
-    float xo[8], yo[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float co = cs[d0 + j], si = cs[half + d0 + j];
-      xo[j] = x.f(j) * co - y.f(j) * si;
-      yo[j] = y.f(j) * co + x.f(j) * si;
-    }
-    *reinterpret_cast<uint4*>(base + d0) = pack_bf16x8(xo);
-    *reinterpret_cast<uint4*>(base + half + d0) = pack_bf16x8(yo);
-  }
-
-  // ---- rotate k (in place) + append to k_cache ----
   const long cache_tok_base =
       slot >= 0 ? ((long)(slot / BS) * Hk * BS + (long)(slot % BS)) * D : 0;
-  const int k_chunks = Hk * (D / 16);
-  for (int c = yoff; c < k_chunks; c += ystride) {
-    const int h = c / (D / 16);
-    const int d0 = (c % (D / 16)) * 8;
-    unsigned short* base = row + (long)(Hq + h) * D;
-    bf16x8 x = load_bf16x8(base + d0);
-    bf16x8 y = load_bf16x8(base + half + d0);
-    float xo[8], yo[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float co = cs[d0 + j], si = cs[half + d0 + j];
-      xo[j] = x.f(j) * co - y.f(j) * si;
-      yo[j] = y.f(j) * co + x.f(j) * si;
-    }
-    uint4 px = pack_bf16x8(xo), py = pack_bf16x8(yo);
-    *reinterpret_cast<uint4*>(base + d0) = px;
-    *reinterpret_cast<uint4*>(base + half + d0) = py;
-    if (slot >= 0) {
-      const long off = cache_tok_base + (long)h * BS * D;
-      if (FP8) {
-        unsigned char* kc = reinterpret_cast<unsigned char*>(k_cache) + off;
-        *reinterpret_cast<uint2*>(kc + d0) = pack_fp8x8(xo);
-        *reinterpret_cast<uint2*>(kc + half + d0) = pack_fp8x8(yo);
-      } else {
-        unsigned short* kc = reinterpret_cast<unsigned short*>(k_cache) + off;
-        *reinterpret_cast<uint4*>(kc + d0) = px;
-        *reinterpret_cast<uint4*>(kc + half + d0) = py;
-      }
-    }
-  }
 
-  // ---- copy v to v_cache ----
-  if (slot >= 0) {
-    const int v_chunks = Hk * (D / 8);
-    for (int c = yoff; c < v_chunks; c += ystride) {
-      const int h = c / (D / 8);
-      const int d0 = (c % (D / 8)) * 8;
-      const unsigned short* base = row + (long)(Hq + Hk + h) * D;
-      const long off = cache_tok_base + (long)h * BS * D;
-      if (FP8) {
-        bf16x8 v = load_bf16x8(base + d0);
-        float f[8];
+  auto load8 = [&](int col, float* f) {
+    if (SUMS) {
+      const float* p = sums + t * row_stride + col;
+      const long slab = (long)gridDim.x * row_stride;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = v.f(j);
-        unsigned char* vc = reinterpret_cast<unsigned char*>(v_cache) + off;
-        *reinterpret_cast<uint2*>(vc + d0) = pack_fp8x8(f);
-      } else {
-        unsigned short* vc = reinterpret_cast<unsigned short*>(v_cache) + off;
-        *reinterpret_cast<uint4*>(vc + d0) =
-            *reinterpret_cast<const uint4*>(base + d0);
+      for (int j = 0; j < 8; ++j) f[j] = 0.f;
+#pragma unroll 4
+      for (int s = 0; s < splits; ++s) {
+        const float4 a = *reinterpret_cast<const float4*>(p + s * slab);
+        const float4 b = *reinterpret_cast<const float4*>(p + s * slab + 4);
+        f[0] += a.x; f[1] += a.y; f[2] += a.z; f[3] += a.w;
+        f[4] += b.x; f[5] += b.y; f[6] += b.z; f[7] += b.w;
       }
+    } else {
+      const bf16x8 v = load_bf16x8(row + col);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = v.f(j);
+    }
+  };
+  auto page_write = [&](void* cache, long off, const float* f, uint4 packed) {
+    if (FP8)
+      *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(cache) +
+                                off) = pack_fp8x8(f);
+    else
+      *reinterpret_cast<uint4*>(reinterpret_cast<unsigned short*>(cache) +
+                                off) = packed;
+  };
+
+  const int pair_chunks = D / 16;                  // per head
+  const int k_first = Hq * pair_chunks;
+  const int v_first = k_first + Hk * pair_chunks;
+  const int total = v_first + Hk * (D / 8);
+  for (int c = yoff; c < total; c += ystride) {
+    if (c < v_first) {
+      const int h = c / pair_chunks;               // keys follow the queries
+      const int d0 = (c % pair_chunks) * 8;
+      float x[8], y[8], xo[8], yo[8];
+      load8(h * D + d0, x);
+      load8(h * D + half + d0, y);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float co = cs[d0 + j], si = cs[half + d0 + j];
+        xo[j] = x[j] * co - y[j] * si;
+        yo[j] = y[j] * co + x[j] * si;
+      }
+      const uint4 px = pack_bf16x8(xo), py = pack_bf16x8(yo);
+      if (!SUMS || c < k_first) {
+        *reinterpret_cast<uint4*>(row + (long)h * D + d0) = px;
+        *reinterpret_cast<uint4*>(row + (long)h * D + half + d0) = py;
+      }
+      if (c >= k_first && slot >= 0) {
+        const long off = cache_tok_base + (long)(h - Hq) * BS * D;
+        page_write(k_cache, off + d0, xo, px);
+        page_write(k_cache, off + half + d0, yo, py);
+      }
+    } else if (slot >= 0) {
+      const int h = (c - v_first) / (D / 8);
+      const int d0 = ((c - v_first) % (D / 8)) * 8;
+      float f[8];
+      load8((Hq + Hk + h) * D + d0, f);
+      page_write(v_cache, cache_tok_base + (long)h * BS * D + d0, f,
+                 pack_bf16x8(f));
     }
   }
 }
 
-void rope_kv_append(torch::Tensor qkv, torch::Tensor k_cache,
-                    torch::Tensor v_cache, torch::Tensor cos_sin,
-                    torch::Tensor positions, torch::Tensor slot_mapping,
-                    int64_t num_q_heads, int64_t num_kv_heads,
-                    int64_t head_dim, torch::Tensor block_table) {
+// `sums`: undefined, or the projection's parts
+static void rope_kv(torch::Tensor qkv, const torch::Tensor& sums,
+                    torch::Tensor k_cache, torch::Tensor v_cache,
+                    torch::Tensor cos_sin, torch::Tensor positions,
+                    torch::Tensor slot_mapping, int64_t num_q_heads,
+                    int64_t num_kv_heads, int64_t head_dim,
+                    torch::Tensor block_table) {
   TORCH_CHECK(qkv.is_contiguous() && qkv.scalar_type() == torch::kBFloat16);
   TORCH_CHECK(cos_sin.scalar_type() == torch::kFloat32);
   TORCH_CHECK(positions.scalar_type() == torch::kInt32);
@@ -144,10 +145,45 @@ void rope_kv_append(torch::Tensor qkv, torch::Tensor k_cache,
   const int mb = table_mode ? (int)block_table.size(1) : 0;
   const bool fp8 = k_cache.scalar_type() == torch::kUInt8;
   const unsigned ysplit = T <= 128 ? 4 : 1;
-#define RK_LAUNCH(FP8_)                                                         rope_kv_kernel<FP8_><<<dim3((unsigned)T, ysplit), 256, 0, stream>>>(              reinterpret_cast<unsigned short*>(qkv.data_ptr()), k_cache.data_ptr(),        v_cache.data_ptr(), cos_sin.data_ptr<float>(),                                positions.data_ptr<int>(), slot_mapping.data_ptr<int>(), bt, mb,              (int)num_q_heads, (int)num_kv_heads, D, BS)
-  if (fp8) { RK_LAUNCH(true); } else { RK_LAUNCH(false); }
+  const bool parts = sums.defined();
+  const float* sp = parts ? sums.data_ptr<float>() : nullptr;
+  const int splits = parts ? (int)sums.size(0) : 0;
+#define RK_LAUNCH(FP8_, SUMS_)                                               \
+  rope_kv_kernel<FP8_, SUMS_><<<dim3((unsigned)T, ysplit), 256, 0, stream>>>(\
+      reinterpret_cast<unsigned short*>(qkv.data_ptr()), sp, splits,         \
+      k_cache.data_ptr(), v_cache.data_ptr(), cos_sin.data_ptr<float>(),     \
+      positions.data_ptr<int>(), slot_mapping.data_ptr<int>(), bt, mb,       \
+      (int)num_q_heads, (int)num_kv_heads, D, BS)
+  if (parts) {
+    if (fp8) { RK_LAUNCH(true, true); } else { RK_LAUNCH(false, true); }
+  } else {
+    if (fp8) { RK_LAUNCH(true, false); } else { RK_LAUNCH(false, false); }
+  }
 #undef RK_LAUNCH
   HIP_CHECK_KERNEL();
+}
+
+void rope_kv_append(torch::Tensor qkv, torch::Tensor k_cache,
+                    torch::Tensor v_cache, torch::Tensor cos_sin,
+                    torch::Tensor positions, torch::Tensor slot_mapping,
+                    int64_t num_q_heads, int64_t num_kv_heads,
+                    int64_t head_dim, torch::Tensor block_table) {
+  rope_kv(qkv, torch::Tensor(), k_cache, v_cache, cos_sin, positions,
+          slot_mapping, num_q_heads, num_kv_heads, head_dim, block_table);
+}
+
+// The projection qkv = x W^T and rope_kv_append in one: the projection's parts
+// go straight to the rotary kernel. Only the query columns of qkv are written.
+void qkv_rope_append(torch::Tensor qkv, torch::Tensor x, torch::Tensor w,
+                     torch::Tensor k_cache, torch::Tensor v_cache,
+                     torch::Tensor cos_sin, torch::Tensor positions,
+                     torch::Tensor slot_mapping, int64_t num_q_heads,
+                     int64_t num_kv_heads, int64_t head_dim,
+                     torch::Tensor block_table) {
+  TORCH_CHECK(qkv.dim() == 2 && qkv.size(0) == x.size(0) &&
+              qkv.size(1) == w.size(0));
+  rope_kv(qkv, stream_gemm_sums(x, w), k_cache, v_cache, cos_sin, positions,
+          slot_mapping, num_q_heads, num_kv_heads, head_dim, block_table);
 }
 
 }  // namespace kukeon

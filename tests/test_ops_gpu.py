@@ -909,3 +909,118 @@ def test_modelhub_server_gpu_streaming():
             assert r2["context_len"] > 8  # persistent multi-turn KV
     finally:
         hub.stop()
+
+
+# ---- weight-streaming products of decode batches ---------------------------
+def _close(got, want, scale):
+    """bf16 rounding of the result (2^-8 of it, half an ulp with room) and
+    fp32 sums of K products of the given scale."""
+    err = (got.double() - want).abs()
+    assert bool((err <= want.abs() * 2.0 ** -8 + scale).all()), \
+        float((err - want.abs() * 2.0 ** -8).max())
+
+
+# row tiles of x (16), units of W (128 rows, 256 columns), one part and many
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 49, 64])
+@pytest.mark.parametrize("N,K", [(128, 256), (256, 768), (2048, 4096),
+                                 (24576, 512), (51200, 256)])
+def test_stream_gemm(M, N, K):
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(N, K, dtype=torch.bfloat16, device=DEV) * K ** -0.5
+    want = x.double() @ w.double().t()
+    out = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._C.stream_gemm(out[:M], x, w)
+    _close(out[:M], want, 1e-5)
+    assert bool((out[M] == 7).all())
+
+    gate, up = want[:, : N // 2], want[:, N // 2:]
+    act = torch.full((M + 1, N // 2), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops._C.stream_gemm_silu(act[:M], x, w)
+    _close(act[:M], torch.nn.functional.silu(gate) * up, 4e-5)
+    assert bool((act[M] == 7).all())
+
+
+@pytest.mark.parametrize("M", [1, 16, 40, 64])
+@pytest.mark.parametrize("N,K", [(2048, 512), (4096, 1024), (8192, 256)])
+def test_stream_gemm_norm(M, N, K):
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(N, K, dtype=torch.bfloat16, device=DEV) * K ** -0.5
+    res = torch.randn(M, N, dtype=torch.bfloat16, device=DEV)
+    nw = torch.randn(N, dtype=torch.bfloat16, device=DEV)
+    want = res.double() + x.double() @ w.double().t()
+    normed = torch.empty_like(res)
+    ops._C.stream_gemm_norm(normed, x, w, res, nw, 1e-5)
+    _close(res, want, 1e-5)
+    # the norm is that of the rounded residual
+    r = res.double()
+    want = r * torch.rsqrt(r.pow(2).mean(-1, keepdim=True) + 1e-5) \
+        * nw.double()
+    _close(normed, want, 1e-5)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("decode", [False, True])
+@pytest.mark.parametrize("T,Hq,Hk,K", [(1, 32, 8, 4096), (37, 8, 8, 4096),
+                                       (64, 14, 1, 8192)])
+def test_qkv_rope_append(T, Hq, Hk, K, decode, fp8):
+    """Against the projection and the rotary kernel one after the other."""
+    torch.manual_seed(T)
+    D, BS = 128, 16
+    N = (Hq + 2 * Hk) * D
+    x = torch.randn(T, K, dtype=torch.bfloat16, device=DEV)
+    w = torch.randn(N, K, dtype=torch.bfloat16, device=DEV) * K ** -0.5
+    i32 = dict(dtype=torch.int32, device=DEV)
+    pos = torch.randint(0, 64, (T,), **i32)
+    if decode and T > 2:
+        pos[1] = -1                       # an inactive row
+    table = torch.arange(T * 4, **i32).view(T, 4) if decode else None
+    slots = torch.arange(T, **i32) * 64 + pos
+    if T > 2 and not decode:
+        slots[2] = -1                     # rotated, but not kept
+    cs = torch.randn(64, D, dtype=torch.float32, device=DEV)
+    dt = torch.uint8 if fp8 else torch.bfloat16
+    kc, vc, kr, vr = (torch.zeros(T * 4, Hk, BS, D, dtype=dt, device=DEV)
+                      for _ in range(4))
+    assert ops._stream_ok(x, w)
+    got = ops.qkv_rope_append(x, w, kc, vc, cs, pos, slots, Hq, Hk, D, table)
+    want = torch.nn.functional.linear(x, w)
+    ops.rope_kv_append(want, kr, vr, cs, pos, slots, Hq, Hk, D, table)
+    live = pos >= 0
+
+    def wide(t):
+        return t.view(torch.float8_e4m3fn).float() if fp8 else t.float()
+
+    # the reference rounds the projection to bf16 first: 2^-8 of |x| + |y|
+    # times |cos|, |sin| (up to about 4), and one more rounding
+    torch.testing.assert_close(got[live, : Hq * D].float(),
+                               want[live, : Hq * D].float(), rtol=2 ** -7,
+                               atol=0.1)
+    # fp8: the two may land on neighbouring values, 2^-3 apart
+    tol = dict(rtol=2 ** -3, atol=0.1) if fp8 else dict(rtol=2 ** -7,
+                                                        atol=0.1)
+    torch.testing.assert_close(wide(kc), wide(kr), **tol)
+    torch.testing.assert_close(wide(vc), wide(vr), **tol)
+
+
+def test_stream_dispatch():
+    """ops.linear takes the streaming kernel for plain decode batches only."""
+    w = torch.randn(4096, 2048, dtype=torch.bfloat16, device=DEV) * 0.02
+    x = torch.randn(64, 2048, dtype=torch.bfloat16, device=DEV)
+    assert ops._stream_ok(x, w)
+    _close(ops.linear(x[:16], w), x[:16].double() @ w.double().t(), 1e-5)
+    wide = torch.randn(64, 4096, dtype=torch.bfloat16, device=DEV)
+    xg = x.clone().requires_grad_()
+    for xx, ww in ((wide[:, :2048], w), (torch.cat([x, x[:1]]), w),
+                   (x[:0], w), (x[:, :1984].contiguous(),
+                                w[:, :1984].contiguous()),
+                   (x, w[:4000].contiguous()), (xg, w), (x.float(), w.float()),
+                   (wide.view(-1)[1: 1 + 64 * 2048].view(64, 2048), w)):
+        assert not ops._stream_ok(xx, ww)
+        torch.testing.assert_close(ops.linear(xx, ww),
+                                   torch.nn.functional.linear(xx, ww))
+    y = torch.vmap(lambda r: ops.linear(r, w))(x.view(4, 16, 2048))
+    torch.testing.assert_close(y.view(64, -1).float(),
+                               torch.nn.functional.linear(x, w).float(),
+                               rtol=1e-2, atol=1e-2)
