@@ -162,10 +162,6 @@ class LLMEngine:
         self.d_seed = torch.full((1,), ecfg.seed, dtype=torch.int64, device=d)
         self.d_ws = torch.zeros(self.Bmax, 528, dtype=torch.float32,
                                 device=d)  # sampling workspace rows
-        # 32 split slots: small decode batches (16-session / 70B configs)
-        # need B*Hk*S ~ 4096 wave-units to fill the MFMA attention kernel
-        # at its 4-waves/SIMD occupancy; 16 capped them at half the chip
-        self.max_splits = 32
         self.d_tmp_out = {}
         self.d_tmp_ml = {}
         # self-advancing decode: token ring + device step counter
@@ -566,16 +562,13 @@ class LLMEngine:
         return self.Bmax
 
     def _decode_splits(self, bucket: int) -> int:
-        # target ~8x the 256 CUs in workgroups: the micro-bench
-        # (scripts/bench_paged_attn.py) shows 2048-4096 WGs runs 5-9%
-        # faster than the 512-WG minimum (imbalance absorption across
-        # the 8 XCDs), flat beyond
-        # target ~4096 split-units: the MFMA decode kernel runs B*Hk*S
-        # autonomous waves (4 per workgroup), and 4096 exactly fills the
-        # chip at its 4-waves/SIMD occupancy (multiple of 4 required —
-        # each workgroup's waves own consecutive split slots)
-        want = (16 * 256 + bucket * self.hk - 1) // (bucket * self.hk)
-        return max(4, min(self.max_splits, ((want + 3) // 4) * 4))
+        # The decode kernel cuts all sequences into pieces of equal length,
+        # about 4096 in all (16 waves on each of the 256 CUs); this is the
+        # most pieces that one sequence may have. A long one among short
+        # ones, or a few alone, need many to fill the chip (one session of
+        # 3500 tokens: 18 us with 16 pieces, 14 with 32, 12 with 64); more
+        # slots than that are only more for the merge to look through.
+        return 32 if bucket * self.hk <= 64 else 16
 
     def _tmp_for(self, bucket: int, splits: int):
         key = (bucket, splits)

@@ -597,23 +597,90 @@ void mfma_probe16k(torch::Tensor out, torch::Tensor a, torch::Tensor b) {
 }
 
 // ===================================================================
-// 16-token-tile MFMA decode attention: the residency-first variant.
+// 16-token-tile MFMA decode attention: the default.
 //
-// Same wave-autonomous split-slot scheme as paged_attn_mfma_kernel, but
-// one cache block (16 tokens) per tile on 16x16 MFMAs:
-//   - S^T[tok, head] via 16x16x32 (K = head_dim chunks),
-//   - PV O^T[d, head] via 16x16x16bf16_1k (K = the 16 tokens) — and in
-//     this swapped shape the C layout of the scores IS the B layout of
-//     P (row=k=4*(l>>4)+idx, col=head), so P needs NO cross-lane
-//     redistribution at all, just two v_cvt_pk_bf16_f32.
-//   - 8 KiB LDS per wave (32 KiB/WG) -> ~5 workgroups/CU, matching the
-//     v_dot2 kernel's residency while issuing ~5x fewer instructions.
-// G <= 16 (8B: 4, 70B: 8); q-head padding is per-lane garbage, never
-// written back.
+// Wave-autonomous split slots as in paged_attn_mfma_kernel, one cache page (16
+// tokens) per tile on 16x16 MFMAs:
+//   - S^T[tok, head] via 16x16x32 (K = head_dim chunks), K consumed from HBM in
+//     fragment shape;
+//   - PV O^T[d, head] via 16x16x16bf16_1k (K = the 16 tokens): in this swapped
+//     shape the C layout of the scores IS the B layout of P
+//     (row=k=4*(l>>4)+idx, col=head), so P needs no cross-lane
+//     redistribution, just two v_cvt_pk_bf16_f32; V lies row-major in 4 KB of
+//     LDS per wave and ds_read_b64_tr_b16 hands each lane its four tokens.
+// What bounds it is the K/V stream from HBM, so what counts is bytes in flight:
+// the next tile's K AND V are in registers' way during the whole of this
+// tile's arithmetic (8 KB per wave, 16 waves per CU), their page ids one tile
+// earlier still, and nothing waits on LDS stores of its own tile but the PV
+// product. (Before, each tile fetched its V, waited for it and stored it
+// transposed, 16 ways into one bank.)
+// Work is shared out by length: all sequences are cut into pieces of the same
+// number of pages, one per wave, about 16 waves for each of 256 CUs; a sequence
+// fills as many of its S slots as it needs. The waves of the grid count the
+// pieces through (every wave does the same short sum over the lengths, which
+// only the device knows), so that no workgroup is empty before the last one.
+// (With S equal pieces per sequence the longest ones' pieces were what the
+// others waited for.)
+// G <= 16 (8B: 4, 70B: 8); q-head padding is per-lane garbage, never written
+// back.
+// Measured with the merge (32 heads on 8, us, before -> now): 64 sequences of
+// 779 to 3466 tokens 160 -> 107 (5.2 TB/s), with the fp8 cache 152 -> 64, 200 of
+// 63 to 751 105 -> 77, one of 3500 34 -> 14, one of 3500 beside 63 of 50
+// 138 -> 20; 64 heads on 8, 16 of 970 to 3150 58 -> 36.
+
+// pages per piece, the same for every wave of a launch; B rows, inactive ones
+// (length <= 0) not counted. A sequence's last piece is rarely a full one: the
+// room for 4096 waves is aimed at with a quarter of a piece per sequence to
+// spare.
+DEV_INLINE int pages_per_slot(const int* __restrict__ seq_lens, int B, int Hk,
+                              int S) {
+  int total = 0, most = 0;
+  for (int i = threadIdx.x & (WAVE - 1); i < B; i += WAVE) {
+    const int pages = (max(seq_lens[i], 0) + 15) / 16;
+    total += pages;
+    most = max(most, pages);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    total += __shfl_xor(total, off, WAVE);
+    most = max(most, __shfl_xor(most, off, WAVE));
+  }
+  const int room = max(4096 - B * Hk / 4, 2048);
+  return __builtin_amdgcn_readfirstlane(
+      max(max((total * Hk + room - 1) / room, (most + S - 1) / S), 1));
+}
+
+// The row and slot of piece j; false past the last piece.
+DEV_INLINE bool find_piece(const int* __restrict__ seq_lens, int B,
+                           int per_slot, int j, int* row, int* slot) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  for (int b0 = 0; b0 < B; b0 += WAVE) {
+    const int len = b0 + lane < B ? max(seq_lens[b0 + lane], 0) : 0;
+    const int n = ((len + 15) / 16 + per_slot - 1) / per_slot;
+    int upto = n;      // pieces of the rows up to and including this lane's
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+      const int v = __shfl_up(upto, off, WAVE);
+      if (lane >= off) upto += v;
+    }
+    const unsigned long long past = __ballot(upto > j);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      *row = b0 + at;
+      *slot = j - __builtin_amdgcn_readlane(upto - n, at);
+      return true;
+    }
+    j -= __builtin_amdgcn_readlane(upto, WAVE - 1);
+  }
+  return false;
+}
+
+typedef __attribute__((address_space(3))) bf16x4_v lds_bf16x4_v;
+typedef __attribute__((__vector_size__(4 * sizeof(unsigned int)))) unsigned int
+    u32x4_v;
+
 template <bool FP8>
-// fp8 needs headroom for the cvt_pk conversions (at 4 waves/SIMD the
-// 128-reg bound put a 2-VGPR spill in the hot loop)
-__global__ __launch_bounds__(256, FP8 ? 3 : 4) void paged_attn_mfma16_kernel(
+__global__ __launch_bounds__(256, 4) void paged_attn_mfma16_kernel(
     float* __restrict__ tmp_out,          // [B, Hq, S, D] f32
     float* __restrict__ tmp_ml,           // [B, Hq, S, 2]
     const unsigned short* __restrict__ q, // [B, q_stride]
@@ -621,36 +688,30 @@ __global__ __launch_bounds__(256, FP8 ? 3 : 4) void paged_attn_mfma16_kernel(
     const void* __restrict__ v_cache,
     const int* __restrict__ block_table,  // [B, max_blocks]
     const int* __restrict__ seq_lens,     // [B]
-    long q_stride, int Hq, int Hk, int max_blocks, int S, float scale) {
+    long q_stride, int B, int Hq, int Hk, int max_blocks, int S,
+    float scale) {
   constexpr int D = 128;
   constexpr int BS = 16;
-  const int b = blockIdx.x;
-  const int hk = blockIdx.y;
-  const int wid = threadIdx.x / WAVE;
+  constexpr float NONE = -3.0e38f;   // running maximum before any key
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x & (WAVE - 1);
   const int g4 = lane >> 4;       // 0..3
   const int rc = lane & 15;
   const int G = Hq / Hk;
-  const int slot = blockIdx.z * 4 + wid;
+  const int piece = blockIdx.x * 4 + wid;
+  const int hk = piece % Hk;
+  const int per_slot = pages_per_slot(seq_lens, B, Hk, S);
+  int b, slot;
+  if (!find_piece(seq_lens, B, per_slot, piece / Hk, &b, &slot)) return;
   const int ctx = seq_lens[b];
-  if (ctx <= 0 || slot >= S) return;
 
-  // V^T images only — K is consumed straight from HBM in fragment shape
-  // (16 B/lane across 64 B-line groups; the LDS round trip was pure
-  // added latency here: per-wave parked time was 67% of cycles). Two
-  // V^T buffers per wave: tile bi's image is written during tile bi-1,
-  // so PV never waits on fresh LDS stores.
-  __shared__ __align__(16) unsigned short vtbuf[4][2][D * BS];
-
-  const int nblocks = (ctx + BS - 1) / BS;
-  const int per_slot = (nblocks + S - 1) / S;
-  const int blk_begin = slot * per_slot;
-  const int blk_end = min(nblocks, blk_begin + per_slot);
-  const int kv_hi = min(ctx, blk_end * BS);
+  __shared__ __align__(16) unsigned short vbuf[4][BS * D];
+  char* vb = reinterpret_cast<char*>(vbuf[wid]);
 
   const int qh = min(rc, G - 1);  // B col = q head
-  // Q fragments pinned in 16 registers (L2 re-reads in the tile loop
-  // measured as 4 dependent ~250-cycle stalls per tile)
+  // a negative scale is a positive one on negated queries
+  const unsigned int flip = scale < 0.f ? 0x80008000u : 0u;
+  const float c2 = fabsf(scale) * 1.44269504088896340736f;
   unsigned int qf[4][4];
   {
     const unsigned short* qp =
@@ -658,173 +719,219 @@ __global__ __launch_bounds__(256, FP8 ? 3 : 4) void paged_attn_mfma16_kernel(
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
       const uint4 v = *reinterpret_cast<const uint4*>(qp + st * 32 + g4 * 8);
-      qf[st][0] = v.x; qf[st][1] = v.y; qf[st][2] = v.z; qf[st][3] = v.w;
+      qf[st][0] = v.x ^ flip; qf[st][1] = v.y ^ flip;
+      qf[st][2] = v.z ^ flip; qf[st][3] = v.w ^ flip;
     }
   }
+  const int pages = (ctx + BS - 1) / BS;
+  const int first = slot * per_slot;
+  const int last = min(pages, first + per_slot) - 1;
+  const int* table = block_table + (long)b * max_blocks;
 
-  float m = -INFINITY, l_acc = 0.f;
+  float mc = NONE, l_acc = 0.f;   // running maximum times c2; lane's sum
   f32x4_v oacc[8] = {{}, {}, {}, {}, {}, {}, {}, {}};
 
-  const unsigned short* kc16 =
-      reinterpret_cast<const unsigned short*>(k_cache);
-  const unsigned short* vc16 =
-      reinterpret_cast<const unsigned short*>(v_cache);
-  const unsigned char* kc8 = reinterpret_cast<const unsigned char*>(k_cache);
-  const unsigned char* vc8 = reinterpret_cast<const unsigned char*>(v_cache);
-
-  // K in MFMA A-fragment shape: lane (rc = token, g4 = k-group) reads
-  // 16 B at tok*256B + st*64B + g4*16B — lanes sharing a token cover one
-  // 64 B line, so the four per-tile loads coalesce at line granularity.
-  uint4 kfr[4];
-  auto kfetch = [&](int bi_f) {
-    const long base =
-        ((long)block_table[(long)b * max_blocks + bi_f] * Hk + hk) * BS * D;
-    const long off = base + (long)rc * D + g4 * 8;
+  // K in MFMA A-fragment shape: lane (rc = token, g4 = k-group) reads 16 B at
+  // tok*256B + st*64B + g4*16B; V in whole rows, four to an instruction
+  uint4 kf[4], vr[4];
+  auto fetch = [&](int page) {
+    const long base = ((long)page * Hk + hk) * BS * D;
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
+      const long ko = base + rc * D + st * 32 + g4 * 8;
+      const long vo = base + (st * 4 + g4) * D + rc * 8;
       if (FP8) {
-        kfr[st] = fp8x8_to_bf16x8(
-            *reinterpret_cast<const uint2*>(kc8 + off + st * 32));
+        const uint2 k8 = *reinterpret_cast<const uint2*>(
+            reinterpret_cast<const unsigned char*>(k_cache) + ko);
+        const uint2 v8 = *reinterpret_cast<const uint2*>(
+            reinterpret_cast<const unsigned char*>(v_cache) + vo);
+        kf[st].x = k8.x; kf[st].y = k8.y;
+        vr[st].x = v8.x; vr[st].y = v8.y;
       } else {
-        kfr[st] = *reinterpret_cast<const uint4*>(kc16 + off + st * 32);
-      }
-    }
-  };
-  const int stg_d0 = rc * 8;
-  uint4 vpre[2][2];
-  auto vfetch = [&](int bi_f) {
-    const long base =
-        ((long)block_table[(long)b * max_blocks + bi_f] * Hk + hk) * BS * D;
-#pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-      const int kp = pass * 4 + g4;
-      const long voff0 = base + (long)(2 * kp) * D + stg_d0;
-      const long voff1 = base + (long)(2 * kp + 1) * D + stg_d0;
-      if (FP8) {
-        vpre[pass][0] =
-            fp8x8_to_bf16x8(*reinterpret_cast<const uint2*>(vc8 + voff0));
-        vpre[pass][1] =
-            fp8x8_to_bf16x8(*reinterpret_cast<const uint2*>(vc8 + voff1));
-      } else {
-        vpre[pass][0] = *reinterpret_cast<const uint4*>(vc16 + voff0);
-        vpre[pass][1] = *reinterpret_cast<const uint4*>(vc16 + voff1);
-      }
-    }
-  };
-  auto vwrite = [&](unsigned short* vt, int kvbase) {
-#pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-      const int kp = pass * 4 + g4;
-      uint4 r0 = vpre[pass][0];
-      uint4 r1 = vpre[pass][1];
-      if (kvbase + 2 * kp >= kv_hi) r0 = uint4{0, 0, 0, 0};
-      if (kvbase + 2 * kp + 1 >= kv_hi) r1 = uint4{0, 0, 0, 0};
-      const unsigned int* a0 = reinterpret_cast<const unsigned int*>(&r0);
-      const unsigned int* a1 = reinterpret_cast<const unsigned int*>(&r1);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const unsigned short e0 = (a0[j >> 1] >> ((j & 1) * 16)) & 0xffffu;
-        const unsigned short e1 = (a1[j >> 1] >> ((j & 1) * 16)) & 0xffffu;
-        const unsigned int packed = (unsigned)e0 | ((unsigned)e1 << 16);
-        const int d = stg_d0 + j;
-        const int byte = d * 32 + ((4 * kp) ^ ((d & 3) << 3));
-        *reinterpret_cast<unsigned int*>(
-            reinterpret_cast<char*>(vt) + byte) = packed;
+        kf[st] = *reinterpret_cast<const uint4*>(
+            reinterpret_cast<const unsigned short*>(k_cache) + ko);
+        // whole lines, used once: no reason to keep them (5.29 against 4.84
+        // TB/s; K's half lines are better off kept for their other halves)
+        vr[st] = __builtin_bit_cast(
+            uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4_v*>(
+                       reinterpret_cast<const unsigned short*>(v_cache) +
+                       vo)));
       }
     }
   };
 
-  if (blk_begin < blk_end) {
-    kfetch(blk_begin);
-    vfetch(blk_begin);
-    vwrite(vtbuf[wid][blk_begin & 1], blk_begin * BS);
-  }
-
-  for (int bi = blk_begin; bi < blk_end; ++bi) {
-    const int kvbase = bi * BS;
-    const unsigned short* vt = vtbuf[wid][bi & 1];
-
-    // ---- S^T = K . Q^T from the in-flight K fragments ----
+  fetch(table[first]);
+  int next_page = table[min(first + 1, last)];
+  for (int bi = first; bi <= last; ++bi) {
+    const bool tail = bi == pages - 1;
+    // ---- V rows to LDS (32-byte pieces swizzled with the token) ----
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+      const int tok = st * 4 + g4;
+      uint4 v = FP8 ? fp8x8_to_bf16x8(uint2{vr[st].x, vr[st].y}) : vr[st];
+      // no value of a row past the context: 0 * NaN would poison the sum
+      if (tail && bi * BS + tok >= ctx) v = uint4{0, 0, 0, 0};
+      *reinterpret_cast<uint4*>(vb + tok * 256 +
+                                ((rc * 16) ^ ((tok & 3) << 5))) = v;
+    }
+    // ---- S^T = K . Q^T ----
     f32x4_v sacc = {};
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
+      const uint4 kk = FP8 ? fp8x8_to_bf16x8(uint2{kf[st].x, kf[st].y})
+                           : kf[st];
       sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          as_frag32(kfr[st].x, kfr[st].y, kfr[st].z, kfr[st].w),
+          as_frag32(kk.x, kk.y, kk.z, kk.w),
           as_frag32(qf[st][0], qf[st][1], qf[st][2], qf[st][3]),
           sacc, 0, 0, 0);
     }
-    // K registers are free again: issue the next tile's fragment loads
-    // (they fly under softmax + V staging + PV + the loop turnaround)
-    if (bi + 1 < blk_end) kfetch(bi + 1);
+    // the next tile is under way during everything that follows
+    if (bi < last) {
+      fetch(next_page);
+      next_page = table[min(bi + 2, last)];
+    }
 
     // ---- online softmax (lane holds tokens 4*g4..+3 of its head) ----
-    float sv[4];
-    float tmax = -INFINITY;
+    if (tail) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const bool valid = (kvbase + 4 * g4 + r) < kv_hi;
-      sv[r] = valid ? sacc[r] * scale : -INFINITY;
-      tmax = fmaxf(tmax, sv[r]);
+      for (int r = 0; r < 4; ++r)
+        if (bi * BS + 4 * g4 + r >= ctx) sacc[r] = -INFINITY;
     }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-    const float mn = fmaxf(m, tmax);
-    const float alpha = (m == -INFINITY) ? 0.f : __expf(m - mn);
-    m = mn;
-    float psum = 0.f;
+    float mx = fmaxf(fmaxf(sacc[0], sacc[1]), fmaxf(sacc[2], sacc[3]));
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+    // the maximum only moves when it is passed by 2^8
+    if (__any(fmaf(mx, c2, -mc) > 8.f)) {
+      const float mn = fmaxf(mc, mx * c2);
+      const float alpha = __builtin_amdgcn_exp2f(mc - mn);
+      mc = mn;
+      l_acc *= alpha;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      sv[r] = (sv[r] == -INFINITY) ? 0.f : __expf(sv[r] - mn);
-      psum += sv[r];
+      for (int dc = 0; dc < 8; ++dc)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) oacc[dc][r] *= alpha;
     }
-    psum += __shfl_xor(psum, 16, WAVE);
-    psum += __shfl_xor(psum, 32, WAVE);
-    l_acc = l_acc * alpha + psum;
+    float p[4];
 #pragma unroll
-    for (int dc = 0; dc < 8; ++dc)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) oacc[dc][r] *= alpha;
-
-    // ---- stage NEXT tile's V^T into the other buffer ----
-    if (bi + 1 < blk_end) {
-      vfetch(bi + 1);
-      vwrite(vtbuf[wid][(bi + 1) & 1], (bi + 1) * BS);
-    }
+    for (int r = 0; r < 4; ++r)
+      p[r] = __builtin_amdgcn_exp2f(fmaf(sacc[r], c2, -mc));
+    l_acc += (p[0] + p[1]) + (p[2] + p[3]);
 
     // ---- PV: P is already a 16x16x16 B fragment ----
-    const bf16x4_v pfrag = as_frag16(cvt_pk_bf16d(sv[0], sv[1]),
-                                     cvt_pk_bf16d(sv[2], sv[3]));
+    const bf16x4_v pfrag =
+        as_frag16(cvtpk_bf16(p[0], p[1]), cvtpk_bf16(p[2], p[3]));
+    // lane i of 16 addresses row 4 g4 + (i >> 2), entries 4 (i & 3).. of a
+    // 16-entry piece and receives entry i of rows 4 g4..+3
+    const int row = 4 * g4 + (rc >> 2);
+    const char* vrow = vb + row * 256 + (rc & 3) * 8;
 #pragma unroll
     for (int dc = 0; dc < 8; ++dc) {
-      const int d = dc * 16 + rc;  // A row = output dim
-      const int byte = d * 32 + ((8 * g4) ^ ((d & 3) << 3));
-      const uint2 vf = *reinterpret_cast<const uint2*>(
-          reinterpret_cast<const char*>(vt) + byte);
-      oacc[dc] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-          as_frag16(vf.x, vf.y), pfrag, oacc[dc], 0, 0, 0);
+      const bf16x4_v vf = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_bf16x4_v*)(__attribute__((address_space(3))) void*)(
+              vrow + ((dc * 32) ^ ((row & 3) << 5))));
+      oacc[dc] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vf, pfrag,
+                                                           oacc[dc], 0, 0, 0);
     }
   }
 
   // ---- epilogue ----
+  l_acc += __shfl_xor(l_acc, 16, WAVE);
+  l_acc += __shfl_xor(l_acc, 32, WAVE);
   if (rc >= G) return;
   const int head = hk * G + rc;
   float* top = tmp_out + (((long)b * Hq + head) * S + slot) * D;
 #pragma unroll
-  for (int dc = 0; dc < 8; ++dc) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      top[dc * 16 + 4 * g4 + r] = oacc[dc][r];
-    }
-  }
-  if (g4 == 0) {
-    float* ml = tmp_ml + (((long)b * Hq + head) * S + slot) * 2;
-    ml[0] = m;
-    ml[1] = l_acc;
-  }
+  for (int dc = 0; dc < 8; ++dc)
+    *reinterpret_cast<float4*>(top + dc * 16 + 4 * g4) =
+        float4{oacc[dc][0], oacc[dc][1], oacc[dc][2], oacc[dc][3]};
+  if (g4 == 0)
+    *reinterpret_cast<float2*>(tmp_ml + (((long)b * Hq + head) * S + slot) *
+                                            2) = float2{mc, l_acc};
 }
 
-// Reduce for the MFMA path: every one of the S slots is written on every
-// call (empty ranges write m = -inf), so all are read unconditionally —
+// Sums of the slots in use. 32 threads cover a slot's 128 entries and take
+// every SHARES-th slot, 8 at a time, so that all loads of up to 8 SHARES slots
+// are under way together; the shares are added up in order. Up to 16 slots a
+// wave does a (row, head) by itself (SHARES = 2, four heads per workgroup),
+// beyond that a workgroup does (SHARES = 8). (One slot after the other took
+// 12 us at 32 slots of one session, where a launch alone takes 4; a workgroup
+// per head 13 us more than a wave for 256 rows of 8 slots.)
+template <int SHARES>
+__global__ __launch_bounds__(256) void paged_attn_merge_kernel(
+    unsigned short* __restrict__ out, const float* __restrict__ tmp_out,
+    const float* __restrict__ tmp_ml, const int* __restrict__ seq_lens,
+    int Hq, int Hk, int S) {
+  constexpr int D = 128;
+  constexpr int HEADS = 8 / SHARES;
+  __shared__ __align__(16) float part[SHARES == 8 ? 8 : 1][D + 4];
+  const int b = blockIdx.x;
+  const int group = threadIdx.x / 32;
+  const int share = group % SHARES;
+  const int h = blockIdx.y * HEADS + group / SHARES;
+  const int ctx = seq_lens[b];
+  if (ctx <= 0 || h >= Hq) return;
+  const int per_slot = pages_per_slot(seq_lens, gridDim.x, Hk, S);
+  const int used = ((ctx + 15) / 16 + per_slot - 1) / per_slot;
+  const float2* ml =
+      reinterpret_cast<const float2*>(tmp_ml) + ((long)b * Hq + h) * S;
+  const float* top = tmp_out + (((long)b * Hq + h) * S) * D;
+  const int d = (threadIdx.x & 31) * 4;
+  float m = -3.0e38f;
+  for (int s = threadIdx.x & (WAVE - 1); s < used; s += WAVE)
+    m = fmaxf(m, ml[s].x);
+  float4 acc{0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+  for (int s0 = 0; s0 < used; s0 += 8 * SHARES) {
+    float4 o[8];
+    float2 e[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (i * SHARES >= used - s0) break;
+      const int s = min(s0 + i * SHARES + share, used - 1);
+      e[i] = ml[s];
+      o[i] = *reinterpret_cast<const float4*>(top + (long)s * D + d);
+    }
+    if (s0 == 0) m = wave_max(m);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (s0 + i * SHARES + share >= used) break;
+      const float w = __builtin_amdgcn_exp2f(e[i].x - m);
+      l = fmaf(w, e[i].y, l);
+      acc.x = fmaf(w, o[i].x, acc.x);
+      acc.y = fmaf(w, o[i].y, acc.y);
+      acc.z = fmaf(w, o[i].z, acc.z);
+      acc.w = fmaf(w, o[i].w, acc.w);
+    }
+  }
+  if (SHARES == 2) {
+    acc.x += __shfl_xor(acc.x, 32, WAVE);
+    acc.y += __shfl_xor(acc.y, 32, WAVE);
+    acc.z += __shfl_xor(acc.z, 32, WAVE);
+    acc.w += __shfl_xor(acc.w, 32, WAVE);
+    l += __shfl_xor(l, 32, WAVE);
+    if (share) return;
+  } else {
+    *reinterpret_cast<float4*>(&part[share][d]) = acc;
+    if (d == 0) part[share][D] = l;
+    __syncthreads();
+    if (share) return;
+    acc = float4{0.f, 0.f, 0.f, 0.f};
+    l = 0.f;
+#pragma unroll
+    for (int i = 0; i < SHARES; ++i) {
+      const float4 p = *reinterpret_cast<const float4*>(&part[i][d]);
+      acc.x += p.x; acc.y += p.y; acc.z += p.z; acc.w += p.w;
+      l += part[i][D];
+    }
+  }
+  const float inv = l != 0.f ? 1.f / l : 0.f;
+  *reinterpret_cast<uint2*>(out + ((long)b * Hq + h) * D + d) =
+      uint2{cvtpk_bf16(acc.x * inv, acc.y * inv),
+            cvtpk_bf16(acc.z * inv, acc.w * inv)};
+}
+
+// Reduce for the 32-token MFMA path: every one of the S slots is written on
+// every call (empty ranges write m = -inf), so all are read unconditionally —
 // no per-split block math, no zero-ctx division hazard.
 template <int D>
 __global__ void paged_attn_reduce_all_kernel(
@@ -878,18 +985,10 @@ void paged_attention(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
   auto* op = reinterpret_cast<unsigned short*>(out.data_ptr());
 
   const bool fp8 = k_cache.scalar_type() == torch::kUInt8;
-  // Opt-in (KUKEON_ATTN_MFMA=1): correct and ~5x fewer wave-instructions
-  // per token, but measured 25-30% behind the v_dot2 kernel end to end —
-  // its 64 KiB LDS caps residency at 2 workgroups/CU while the v_dot2
-  // kernel's 8 KiB image keeps ~8x more waves in flight to hide its
-  // issue stalls. Round-2 lever: 16-token tiles on 16x16x32 MFMAs
-  // (quarter the LDS) or a hand-scheduled pipeline.
-  // DEFAULT: the 16-token-tile MFMA kernel (fragment-direct K, double-
-  // buffered V^T, zero barriers) — measured 4.9-5.4 TB/s (78-86% of the
-  // HBM roofline) vs the v_dot2 kernel's 3.8-4.1 on the decode shapes.
-  // KUKEON_ATTN_MFMA=0 forces v_dot2, =32 the 32-token 32x32 variant;
-  // v_dot2 also remains the fallback for split counts not divisible by
-  // 4 and GQA groups over 16.
+  // The 16-token-tile MFMA kernel serves what it can: split counts divisible
+  // by 4 (num_splits is then the most parts a sequence may have) and GQA
+  // groups up to 16. KUKEON_ATTN_MFMA=0 forces v_dot2, =32 the 32-token
+  // variant.
   const char* mfma_env = getenv("KUKEON_ATTN_MFMA");
   const bool want32 = mfma_env && mfma_env[0] == '3' && G <= 32;
   const bool want16 = !want32 && (!mfma_env || mfma_env[0] != '0') && G <= 16;
@@ -900,20 +999,40 @@ void paged_attention(torch::Tensor out, torch::Tensor q, torch::Tensor k_cache,
     dim3 mgrid(B, Hk, (unsigned)(num_splits / 4));
     float* tovm = tmp_out.data_ptr<float>();
     float* tmlm = tmp_ml.data_ptr<float>();
-#define PAM_LAUNCH(KERN, FP8_)                                               \
-    KERN<FP8_><<<mgrid, 256, 0, stream>>>(                                   \
-        tovm, tmlm, qp, k_cache.data_ptr(), v_cache.data_ptr(),              \
-        block_table.data_ptr<int>(), seq_lens.data_ptr<int>(), q_stride,     \
-        Hq, Hk, max_blocks, (int)num_splits, (float)scale)
     if (want16) {
-      if (fp8) { PAM_LAUNCH(paged_attn_mfma16_kernel, true); }
-      else { PAM_LAUNCH(paged_attn_mfma16_kernel, false); }
+      // as many waves as there can be pieces
+      const long most = std::min(4096L + (long)B * Hk,
+                                 (long)B * Hk * num_splits);
+#define PAM_LAUNCH(FP8_)                                                     \
+      paged_attn_mfma16_kernel<FP8_>                                         \
+          <<<(unsigned)((most + 3) / 4), 256, 0, stream>>>(                  \
+          tovm, tmlm, qp, k_cache.data_ptr(), v_cache.data_ptr(),            \
+          block_table.data_ptr<int>(), seq_lens.data_ptr<int>(), q_stride,   \
+          B, Hq, Hk, max_blocks, (int)num_splits, (float)scale)
+      if (fp8) { PAM_LAUNCH(true); } else { PAM_LAUNCH(false); }
+#undef PAM_LAUNCH
     } else {
-      if (fp8) { PAM_LAUNCH(paged_attn_mfma_kernel, true); }
-      else { PAM_LAUNCH(paged_attn_mfma_kernel, false); }
+#define PAM_LAUNCH(FP8_)                                                     \
+      paged_attn_mfma_kernel<FP8_><<<mgrid, 256, 0, stream>>>(               \
+          tovm, tmlm, qp, k_cache.data_ptr(), v_cache.data_ptr(),            \
+          block_table.data_ptr<int>(), seq_lens.data_ptr<int>(), q_stride,   \
+          Hq, Hk, max_blocks, (int)num_splits, (float)scale)
+      if (fp8) { PAM_LAUNCH(true); } else { PAM_LAUNCH(false); }
     }
 #undef PAM_LAUNCH
     HIP_CHECK_KERNEL();
+    if (want16) {
+      if (num_splits <= 16)
+        paged_attn_merge_kernel<2><<<dim3(B, (Hq + 3) / 4), 256, 0, stream>>>(
+            op, tovm, tmlm, seq_lens.data_ptr<int>(), Hq, Hk,
+            (int)num_splits);
+      else
+        paged_attn_merge_kernel<8><<<dim3(B, Hq), 256, 0, stream>>>(
+            op, tovm, tmlm, seq_lens.data_ptr<int>(), Hq, Hk,
+            (int)num_splits);
+      HIP_CHECK_KERNEL();
+      return;
+    }
     dim3 rgrid(B, Hq);
     paged_attn_reduce_all_kernel<128><<<rgrid, 128, 0, stream>>>(
         op, tovm, tmlm, seq_lens.data_ptr<int>(), Hq, (int)num_splits);

@@ -1024,3 +1024,43 @@ def test_stream_dispatch():
     torch.testing.assert_close(y.view(64, -1).float(),
                                torch.nn.functional.linear(x, w).float(),
                                rtol=1e-2, atol=1e-2)
+
+
+# pieces of sequences of very different lengths: none, one token, page edges,
+# one that needs all its slots; rows beyond a wave's 64 lanes; groups of heads
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hk,splits,lens", [
+    (8, 2, 4, [0, 1, 15, 16, 17, 0, 700]),
+    (4, 4, 16, [257, 0, 16 * 16, 16 * 16 + 1]),
+    (16, 1, 8, [5] * 66 + [0, 333, 31]),
+    (8, 1, 32, [1500]),
+    (4, 2, 24, [0, 0, 600]),
+])
+def test_paged_attention_pieces(Hq, Hk, splits, lens, fp8):
+    torch.manual_seed(len(lens))
+    D, B = 128, len(lens)
+    pages = [(n + 15) // 16 for n in lens]
+    kc, vc = _make_cache(sum(pages) + 1, Hk, 16, D, fp8=fp8)
+    bt = torch.zeros(B, max(pages), dtype=torch.int32)
+    order, at = torch.randperm(sum(pages)).int(), 0
+    for i, n in enumerate(pages):
+        bt[i, :n] = order[at: at + n]
+        at += n
+    bt, sl = bt.to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = torch.randn(B, Hq * D, dtype=torch.bfloat16, device=DEV)
+    out = torch.full((B, Hq * D), 7.0, dtype=torch.bfloat16, device=DEV)
+    # what the slots held before does not matter
+    t_o = torch.full((B, Hq, splits, D), float("nan"), device=DEV)
+    t_m = torch.full((B, Hq, splits, 2), float("nan"), device=DEV)
+    ops.paged_attention(out, q, kc, vc, bt, sl, 0, splits, D ** -0.5, t_o,
+                        t_m)
+    live = sl.cpu() > 0
+    ref = torch.full((B, Hq * D), 7.0, dtype=torch.bfloat16)
+    got = torch.empty(int(live.sum()), Hq * D, dtype=torch.bfloat16)
+    reference.paged_attention(got, q.cpu()[live], kc.cpu(), vc.cpu(),
+                              bt.cpu()[live], sl.cpu()[live], 0, 1,
+                              D ** -0.5, None, None)
+    ref[live] = got
+    tol = 7e-2 if fp8 else 2.5e-2
+    torch.testing.assert_close(out.cpu().float(), ref.float(), rtol=tol,
+                               atol=tol)
