@@ -56,13 +56,79 @@ DEV_INLINE float uniform01(unsigned long long seed, unsigned int row,
   return ((h >> 40) + 1.f) * (1.f / 16777217.f);
 }
 
-struct Chunk {
-  int lo, hi;
+// Calls f(index, value) for this thread's share of chunk s of a row. With
+// VEC (rows that start on 16 bytes) a thread takes 8 neighbours per load; a
+// chunk is a multiple of 8 entries either way.
+template <bool VEC, typename F>
+DEV_INLINE void for_chunk(const unsigned short* __restrict__ row, int V,
+                          int splits, int s, F f) {
+  const int per = ((V + splits - 1) / splits + 7) / 8 * 8;
+  const int lo = min(V, s * per), hi = min(V, lo + per);
+  if (VEC) {
+    for (int i = lo + (int)threadIdx.x * 8; i < hi; i += blockDim.x * 8) {
+      const bf16x8 v = load_bf16x8(row + i);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f(i + j, v.us(j));
+    }
+  } else {
+    for (int i = lo + (int)threadIdx.x; i < hi; i += blockDim.x) f(i, row[i]);
+  }
+}
+
+// Histograms in LDS, one copy for every 16th lane: a row's logits fall into a
+// handful of the 256 bins, and with one copy all lanes of a wave queue at the
+// same address (this pass took 212 of the 500 us that 256 rows of 128256 took
+// in all; with copies, wide loads and the walks in LDS all passes take 233, 8
+// rows 33 instead of 50). Copies start 8 banks apart.
+constexpr int COPIES = 16;
+constexpr int COPY = 256 + 8;
+struct Hists {
+  unsigned int count[COPIES * COPY];
+  float weight[COPIES * COPY];
 };
-DEV_INLINE Chunk chunk_of(int V, int splits, int s) {
-  const int per = (V + splits - 1) / splits;
-  Chunk c{s * per, min(V, (s + 1) * per)};
-  return c;
+DEV_INLINE void clear(Hists& h) {
+  for (int i = threadIdx.x; i < COPIES * COPY; i += blockDim.x) {
+    h.count[i] = 0;
+    h.weight[i] = 0.f;
+  }
+}
+DEV_INLINE void merge(const Hists& h, float* wsb) {
+  unsigned int* gc = reinterpret_cast<unsigned int*>(wsb + 16);
+  float* gw = wsb + 272;
+  for (int i = threadIdx.x; i < 256; i += blockDim.x) {
+    unsigned int n = 0;
+    float w = 0.f;
+#pragma unroll
+    for (int c = 0; c < COPIES; ++c) {
+      n += h.count[c * COPY + i];
+      w += h.weight[c * COPY + i];
+    }
+    if (n) atomicAdd(&gc[i], n);
+    if (w != 0.f) atomicAdd(&gw[i], w);
+  }
+}
+
+// From the top bin down, the first at which the sum reaches `need` (or bin 0);
+// *cum gets the sum above it. One thread, in this order (the sums are floats);
+// the bins are in LDS and read 8 at a time, ahead of the additions. (Read
+// from memory one by one they took 10 to 19 us.)
+DEV_INLINE int walk(const float* bins, float need, float* cum) {
+  float sum = 0.f;
+  for (int b0 = 255; b0 >= 0; b0 -= 8) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = bins[b0 - j];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (sum + v[j] >= need || b0 - j == 0) {
+        *cum = sum;
+        return b0 - j;
+      }
+      sum += v[j];
+    }
+  }
+  *cum = sum;
+  return 0;
 }
 
 // ---- K0: zero the workspace rows. A kernel, NOT hipMemsetAsync: a
@@ -74,15 +140,14 @@ __global__ void k0_zero(float* __restrict__ ws) {
 }
 
 // ---- K1: row max (mapped) + invT ----
+template <bool VEC>
 __global__ void k1_max(float* __restrict__ ws,
                        const unsigned short* __restrict__ logits,
                        const float* __restrict__ temps, int V, int splits) {
   const int b = blockIdx.x;
-  const Chunk c = chunk_of(V, splits, blockIdx.y);
-  const unsigned short* row = logits + (long)b * V;
   unsigned int mx = 0;
-  for (int i = c.lo + threadIdx.x; i < c.hi; i += blockDim.x)
-    mx = max(mx, map16(row[i]));
+  for_chunk<VEC>(logits + (long)b * V, V, splits, blockIdx.y,
+                 [&](int, unsigned short us) { mx = max(mx, map16(us)); });
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1)
     mx = max(mx, (unsigned)__shfl_xor((int)mx, off, WAVE));
@@ -101,160 +166,131 @@ __global__ void k1_max(float* __restrict__ ws,
 }
 
 // ---- K2: level-0 histograms (count + exp-weight) + Z ----
+template <bool VEC>
 __global__ void k2_hist0(float* __restrict__ ws,
                          const unsigned short* __restrict__ logits, int V,
                          int splits) {
-  __shared__ unsigned int hc[256];
-  __shared__ float hw[256];
+  __shared__ Hists h;
   __shared__ float redf[16];
   const int b = blockIdx.x;
   float* wsb = ws + (long)b * WS_ROW;
-  const Chunk c = chunk_of(V, splits, blockIdx.y);
-  const unsigned short* row = logits + (long)b * V;
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) {
-    hc[i] = 0;
-    hw[i] = 0.f;
-  }
+  clear(h);
   __syncthreads();
   const float mx = unmap16_f(
       *reinterpret_cast<const unsigned int*>(wsb + 0));
   const float invT = wsb[2];
+  const int copy = (threadIdx.x & (COPIES - 1)) * COPY;
   float z = 0.f;
-  for (int i = c.lo + threadIdx.x; i < c.hi; i += blockDim.x) {
-    const unsigned short us = row[i];
-    const unsigned int mu = map16(us);
-    const float e = __expf((us2f(us) - mx) * invT);
-    z += e;
-    atomicAdd(&hc[mu >> 8], 1u);
-    atomicAdd(&hw[mu >> 8], e);
-  }
+  for_chunk<VEC>(logits + (long)b * V, V, splits, blockIdx.y,
+                 [&](int, unsigned short us) {
+                   const unsigned int mu = map16(us);
+                   const float e = __expf((us2f(us) - mx) * invT);
+                   z += e;
+                   atomicAdd(&h.count[copy + (mu >> 8)], 1u);
+                   if (e != 0.f) atomicAdd(&h.weight[copy + (mu >> 8)], e);
+                 });
   z = block_reduce(z, redf, SumOp{}, 0.f);
   if (threadIdx.x == 0) atomicAdd(wsb + 1, z);
   __syncthreads();
-  unsigned int* gc = reinterpret_cast<unsigned int*>(wsb + 16);
-  float* gw = wsb + 272;
+  merge(h, wsb);
+}
+
+// The 256 counts (as floats) and weights of a row, from memory to LDS.
+DEV_INLINE void stage_bins(const float* wsb, float* counts, float* weights) {
   for (int i = threadIdx.x; i < 256; i += blockDim.x) {
-    if (hc[i]) atomicAdd(&gc[i], hc[i]);
-    if (hw[i] != 0.f) atomicAdd(&gw[i], hw[i]);
+    counts[i] = (float)reinterpret_cast<const unsigned int*>(wsb + 16)[i];
+    weights[i] = wsb[272 + i];
   }
+  __syncthreads();
 }
 
 // ---- K3: walk level 0 for both constraints, then re-zero the hists ----
 __global__ void k3_walk0(float* __restrict__ ws,
                          const int* __restrict__ top_k,
                          const float* __restrict__ top_p, int V) {
+  __shared__ float counts[256], weights[256];
   const int b = blockIdx.x;
   float* wsb = ws + (long)b * WS_ROW;
-  unsigned int* gc = reinterpret_cast<unsigned int*>(wsb + 16);
-  float* gw = wsb + 272;
+  stage_bins(wsb, counts, weights);
+  // the two walks run in different waves
   if (threadIdx.x == 0) {
     const int k = top_k[b];
+    unsigned int sel = 0xffffffffu;
     if (k > 0 && k < V) {
-      float cum = 0.f;
-      int sel = 0;
-      for (int bin = 255; bin >= 0; --bin) {
-        if (cum + (float)gc[bin] >= (float)k || bin == 0) { sel = bin; break; }
-        cum += (float)gc[bin];
-      }
-      *reinterpret_cast<unsigned int*>(wsb + 4) = (unsigned)sel;
+      float cum;
+      sel = (unsigned)walk(counts, (float)k, &cum);
       wsb[8] = (float)k - cum;
-    } else {
-      *reinterpret_cast<unsigned int*>(wsb + 4) = 0xffffffffu;
     }
-  } else if (threadIdx.x == 1) {
+    *reinterpret_cast<unsigned int*>(wsb + 4) = sel;
+  } else if (threadIdx.x == WAVE) {
     const float p = top_p[b];
+    unsigned int sel = 0xffffffffu;
     if (p > 0.f && p < 1.f) {
       const float need = p * wsb[1];
-      float cum = 0.f;
-      int sel = 0;
-      for (int bin = 255; bin >= 0; --bin) {
-        if (cum + gw[bin] >= need || bin == 0) { sel = bin; break; }
-        cum += gw[bin];
-      }
-      *reinterpret_cast<unsigned int*>(wsb + 5) = (unsigned)sel;
+      float cum;
+      sel = (unsigned)walk(weights, need, &cum);
       wsb[9] = need - cum;
-    } else {
-      *reinterpret_cast<unsigned int*>(wsb + 5) = 0xffffffffu;
     }
+    *reinterpret_cast<unsigned int*>(wsb + 5) = sel;
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) {
-    gc[i] = 0;
-    gw[i] = 0.f;
-  }
+  for (int i = threadIdx.x; i < 512; i += blockDim.x) wsb[16 + i] = 0.f;
 }
 
 // ---- K4: level-1 histograms restricted to the selected level-0 bins ----
+template <bool VEC>
 __global__ void k4_hist1(float* __restrict__ ws,
                          const unsigned short* __restrict__ logits, int V,
                          int splits) {
-  __shared__ unsigned int hc[256];
-  __shared__ float hw[256];
+  __shared__ Hists h;
   const int b = blockIdx.x;
   float* wsb = ws + (long)b * WS_ROW;
   const unsigned int pk = *reinterpret_cast<const unsigned int*>(wsb + 4);
   const unsigned int pp = *reinterpret_cast<const unsigned int*>(wsb + 5);
   if (pk == 0xffffffffu && pp == 0xffffffffu) return;
-  const Chunk c = chunk_of(V, splits, blockIdx.y);
-  const unsigned short* row = logits + (long)b * V;
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) {
-    hc[i] = 0;
-    hw[i] = 0.f;
-  }
+  clear(h);
   __syncthreads();
   const float mx = unmap16_f(*reinterpret_cast<const unsigned int*>(wsb));
   const float invT = wsb[2];
-  for (int i = c.lo + threadIdx.x; i < c.hi; i += blockDim.x) {
-    const unsigned short us = row[i];
-    const unsigned int mu = map16(us);
-    const unsigned int hi8 = mu >> 8;
-    if (hi8 == pk) atomicAdd(&hc[mu & 0xffu], 1u);
-    if (hi8 == pp)
-      atomicAdd(&hw[mu & 0xffu], __expf((us2f(us) - mx) * invT));
-  }
+  const int copy = (threadIdx.x & (COPIES - 1)) * COPY;
+  for_chunk<VEC>(logits + (long)b * V, V, splits, blockIdx.y,
+                 [&](int, unsigned short us) {
+                   const unsigned int mu = map16(us);
+                   const unsigned int hi8 = mu >> 8;
+                   if (hi8 == pk)
+                     atomicAdd(&h.count[copy + (mu & 0xffu)], 1u);
+                   if (hi8 == pp)
+                     atomicAdd(&h.weight[copy + (mu & 0xffu)],
+                               __expf((us2f(us) - mx) * invT));
+                 });
   __syncthreads();
-  unsigned int* gc = reinterpret_cast<unsigned int*>(wsb + 16);
-  float* gw = wsb + 272;
-  for (int i = threadIdx.x; i < 256; i += blockDim.x) {
-    if (hc[i]) atomicAdd(&gc[i], hc[i]);
-    if (hw[i] != 0.f) atomicAdd(&gw[i], hw[i]);
-  }
+  merge(h, wsb);
 }
 
 // ---- K5: walk level 1 -> final logit threshold ----
 __global__ void k5_walk1(float* __restrict__ ws, int V) {
+  __shared__ float counts[256], weights[256];
+  __shared__ float th[2];
   const int b = blockIdx.x;
   float* wsb = ws + (long)b * WS_ROW;
-  if (threadIdx.x != 0) return;
-  unsigned int* gc = reinterpret_cast<unsigned int*>(wsb + 16);
-  float* gw = wsb + 272;
   const unsigned int pk = *reinterpret_cast<const unsigned int*>(wsb + 4);
   const unsigned int pp = *reinterpret_cast<const unsigned int*>(wsb + 5);
-  float th = -INFINITY;
-  if (pk != 0xffffffffu) {
-    const float need = wsb[8];
-    float cum = 0.f;
-    int sel = 0;
-    for (int bin = 255; bin >= 0; --bin) {
-      if (cum + (float)gc[bin] >= need || bin == 0) { sel = bin; break; }
-      cum += (float)gc[bin];
-    }
-    th = fmaxf(th, unmap16_f((pk << 8) | (unsigned)sel));
-  }
-  if (pp != 0xffffffffu) {
-    const float need = wsb[9];
-    float cum = 0.f;
-    int sel = 0;
-    for (int bin = 255; bin >= 0; --bin) {
-      if (cum + gw[bin] >= need || bin == 0) { sel = bin; break; }
-      cum += gw[bin];
-    }
-    th = fmaxf(th, unmap16_f((pp << 8) | (unsigned)sel));
-  }
-  wsb[3] = th;
+  stage_bins(wsb, counts, weights);
+  float cum;
+  if (threadIdx.x == 0)
+    th[0] = pk == 0xffffffffu
+                ? -INFINITY
+                : unmap16_f((pk << 8) | (unsigned)walk(counts, wsb[8], &cum));
+  if (threadIdx.x == WAVE)
+    th[1] = pp == 0xffffffffu
+                ? -INFINITY
+                : unmap16_f((pp << 8) | (unsigned)walk(weights, wsb[9],
+                                                       &cum));
+  __syncthreads();
+  if (threadIdx.x == 0) wsb[3] = fmaxf(fmaxf(-INFINITY, th[0]), th[1]);
 }
 
 // ---- K6: masked Gumbel argmax, packed 64-bit atomic merge ----
+template <bool VEC>
 __global__ void k6_draw(float* __restrict__ ws,
                         const unsigned short* __restrict__ logits,
                         const float* __restrict__ temps,
@@ -262,8 +298,6 @@ __global__ void k6_draw(float* __restrict__ ws,
                         int splits) {
   const int b = blockIdx.x;
   float* wsb = ws + (long)b * WS_ROW;
-  const Chunk c = chunk_of(V, splits, blockIdx.y);
-  const unsigned short* row = logits + (long)b * V;
   const float T = temps[b];
   const bool greedy = T <= 0.f;
   const float mx = unmap16_f(*reinterpret_cast<const unsigned int*>(wsb));
@@ -272,18 +306,23 @@ __global__ void k6_draw(float* __restrict__ ws,
   const unsigned long long sd = seed[0];
   float best = -INFINITY;
   int besti = 0;
-  for (int i = c.lo + threadIdx.x; i < c.hi; i += blockDim.x) {
-    const float l = us2f(row[i]);
-    if (l < th) continue;
-    float key;
-    if (greedy) {
-      key = l;
-    } else {
-      key = (l - mx) * invT -
-            __logf(-__logf(uniform01(sd, (unsigned)b, (unsigned)i)));
-    }
-    if (key > best || (key == best && i < besti)) { best = key; besti = i; }
-  }
+  for_chunk<VEC>(
+      logits + (long)b * V, V, splits, blockIdx.y,
+      [&](int i, unsigned short us) {
+        const float l = us2f(us);
+        if (l < th) return;
+        float key;
+        if (greedy) {
+          key = l;
+        } else {
+          key = (l - mx) * invT -
+                __logf(-__logf(uniform01(sd, (unsigned)b, (unsigned)i)));
+        }
+        if (key > best || (key == best && i < besti)) {
+          best = key;
+          besti = i;
+        }
+      });
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     const float ov = __shfl_xor(best, off, WAVE);
@@ -373,23 +412,29 @@ void sample(torch::Tensor tokens, torch::Tensor logits, torch::Tensor temps,
   auto stream = c10::hip::getCurrentHIPStream().stream();
   const auto* lp = reinterpret_cast<const unsigned short*>(logits.data_ptr());
   float* ws = workspace.data_ptr<float>();
-  // fill the chip: ~512 workgroups across the split dimension
-  const int splits = max(1, min(64, 512 / B));
+  // as many workgroups as fit with their histograms (34 KB each, 4 to a CU)
+  const int splits = max(1, min(64, 1024 / B));
   dim3 wide(B, splits);
   k0_zero<<<B, 256, 0, stream>>>(ws);
-  k1_max<<<wide, 256, 0, stream>>>(ws, lp, temps.data_ptr<float>(), V,
-                                   splits);
-  k2_hist0<<<wide, 256, 0, stream>>>(ws, lp, V, splits);
-  k3_walk0<<<B, 256, 0, stream>>>(ws, top_k.data_ptr<int>(),
-                                  top_p.data_ptr<float>(), V);
-  k4_hist1<<<wide, 256, 0, stream>>>(ws, lp, V, splits);
-  k5_walk1<<<B, 64, 0, stream>>>(ws, V);
-  k6_draw<<<wide, 256, 0, stream>>>(
-      ws, lp, temps.data_ptr<float>(),
-      reinterpret_cast<unsigned long long*>(seed.data_ptr()), V, splits);
+  auto* sp = reinterpret_cast<unsigned long long*>(seed.data_ptr());
+#define SAMPLE_PASS(VEC_)                                                    \
+  k1_max<VEC_><<<wide, 256, 0, stream>>>(ws, lp, temps.data_ptr<float>(), V, \
+                                         splits);                            \
+  k2_hist0<VEC_><<<wide, 256, 0, stream>>>(ws, lp, V, splits);               \
+  k3_walk0<<<B, 256, 0, stream>>>(ws, top_k.data_ptr<int>(),                 \
+                                  top_p.data_ptr<float>(), V);               \
+  k4_hist1<VEC_><<<wide, 256, 0, stream>>>(ws, lp, V, splits);               \
+  k5_walk1<<<B, 256, 0, stream>>>(ws, V);                                    \
+  k6_draw<VEC_><<<wide, 256, 0, stream>>>(ws, lp, temps.data_ptr<float>(),   \
+                                          sp, V, splits)
+  if (V % 8 == 0 && reinterpret_cast<uintptr_t>(lp) % 16 == 0) {
+    SAMPLE_PASS(true);
+  } else {
+    SAMPLE_PASS(false);
+  }
+#undef SAMPLE_PASS
   k7_finalize<<<(B + 255) / 256, 256, 0, stream>>>(
-      tokens.data_ptr<int>(), ws,
-      reinterpret_cast<unsigned long long*>(seed.data_ptr()), B);
+      tokens.data_ptr<int>(), ws, sp, B);
   HIP_CHECK_KERNEL();
 }
 

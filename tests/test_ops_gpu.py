@@ -216,6 +216,41 @@ def test_sample_topp_membership():
             assert int(tokens[b]) in allowed[b]
 
 
+# rows that start on 16 bytes (8 logits per load) and rows that do not, chunks
+# that end inside a row, fewer logits than threads
+@pytest.mark.parametrize("B,V", [(1, 8), (2, 7), (3, 1000), (5, 1001),
+                                 (300, 4096), (2, 128256)])
+def test_sample_layouts(B, V):
+    """The same logits in aligned and in shifted rows, under the same seed:
+    the same tokens (top-k counts are whole numbers); greedy is argmax."""
+    torch.manual_seed(V)
+    logits = (torch.randn(B, V) * 3).bfloat16().to(DEV)
+    # no equal largest logits
+    top = torch.randint(0, V, (B, 1), device=DEV)
+    logits.scatter_(1, top, 40.0)
+    shifted = torch.empty(B * V + 1, dtype=torch.bfloat16,
+                          device=DEV)[1:].view(B, V)
+    shifted.copy_(logits)
+    tk = torch.full((B,), 5, dtype=torch.int32, device=DEV)
+    tp = torch.ones(B, dtype=torch.float32, device=DEV)
+    ws = torch.zeros(B, 528, dtype=torch.float32, device=DEV)
+    for temp in (0.0, 30.0):
+        temps = torch.full((B,), temp, dtype=torch.float32, device=DEV)
+        got = []
+        for rows in (logits, shifted):
+            seed = torch.full((1,), 17, dtype=torch.int64, device=DEV)
+            out = torch.full((B,), -1, dtype=torch.int32, device=DEV)
+            ops.sample(out, rows, temps, tk, tp, seed, ws)
+            got.append(out)
+        assert torch.equal(got[0], got[1])
+        if temp == 0.0:
+            assert torch.equal(got[0].long(), top[:, 0])
+        else:
+            kth = logits.float().topk(min(5, V), dim=-1).values[:, -1]
+            chosen = logits.float().gather(1, got[0].long()[:, None])[:, 0]
+            assert bool((chosen >= kth).all())
+
+
 def test_moe_gather_scatter():
     torch.manual_seed(10)
     T, H, K = 13, 4096, 2
