@@ -354,13 +354,13 @@ def _skinny5_wins(rows: int, N: int, K: int) -> bool:
     return N % 2048 == 0 and N <= 8192 and K % 128 == 0 and K >= 3 * N
 
 
-def _stream_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+def _stream_ok(x: torch.Tensor, w: torch.Tensor, most: int = 64) -> bool:
     """Whether x @ w.T goes to the weight-streaming kernel (stream_gemm.hip):
-    a decode batch of up to 64 plain bf16 rows against a matrix of at least
+    a decode batch of up to `most` plain bf16 rows against a matrix of at least
     4 MB (2 MB: 5.6 us against hipBLASLt's 5.8), in the kernel's units of 128
     rows and 256 columns."""
     return (_C is not None and _USE_SKINNY == "0" and x.is_cuda
-            and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= 64
+            and x.dim() == 2 and w.dim() == 2 and 0 < x.shape[0] <= most
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and x.shape[1] == w.shape[1] and w.device == x.device
             and w.shape[0] % 128 == 0 and w.shape[1] % 256 == 0
@@ -383,7 +383,8 @@ def _stream_wins(rows: int, N: int, K: int) -> bool:
     up to 16 rows everywhere (2048 x 2048 8 to 11, 4096 x 1024 7 to 7.5, 6144 x
     4096 15 to 16, 28672 x 4096 45 to 64); with more rows adding the parts up
     costs what the stream gains (6144 x 2048 at 32 rows 13.2 to 12.4), unless
-    the reduction is long (4096 x 14336 28 to 34 at 32 rows, 34 to 41 at 64) or
+    the reduction is long (4096 x 14336 28 to 34 at 32 rows, 34 to 41 at 64,
+    and up to 128 rows) or
     there are enough output columns to need no parts, and not so many that
     hipBLASLt's tiles fill the chip (28672 x 4096 52 to 63 at 48 rows, 32000 x
     8192 106 to 134, but 128256 x 4096 213 to 207)."""
@@ -394,7 +395,7 @@ def _stream_wins(rows: int, N: int, K: int) -> bool:
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear with a weight-streaming kernel on the decode shapes where it
     measured faster than hipBLASLt; hipBLASLt otherwise."""
-    if (_stream_ok(x, w)
+    if (_stream_ok(x, w, 128)
             and _stream_wins(x.shape[0], w.shape[0], w.shape[1])):
         out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,
                           device=x.device)
@@ -475,7 +476,7 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor,
     rows = x.shape[0]
     N, K = w.shape
     if (parallel.tp_size() == 1 and N % 2048 == 0 and N <= 8192
-            and residual.is_contiguous() and _stream_ok(x, w)):
+            and residual.is_contiguous() and _stream_ok(x, w, 128)):
         normed = torch.empty(rows, N, dtype=x.dtype, device=x.device)
         _C.stream_gemm_norm(normed, x, w, residual, norm_weight, eps)
         return normed
@@ -595,7 +596,7 @@ def qkv_rope_append(x: torch.Tensor, w: torch.Tensor, k_cache, v_cache,
     -> [T, (Hq + 2 Hk) D], of which the query columns are meant to be read
     (decode batches leave the others unwritten: keys and values go from the
     projection's fp32 sums straight to their page)."""
-    if _stream_ok(x, w) and head_dim % 16 == 0:
+    if _stream_ok(x, w, 128) and head_dim % 16 == 0:
         if block_table is None:
             block_table = torch.empty(0, dtype=torch.int32, device=x.device)
         qkv = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype,

@@ -1,5 +1,6 @@
 // Weight-streaming matrix products of decode batches for gfx950:
-// y[M, N] = x[M, K] W[N, K]^T, M <= 64, bf16 with fp32 sums.
+// y[M, N] = x[M, K] W[N, K]^T, M <= 64 (128 for partial sums), bf16 with fp32
+// sums.
 //
 // What bounds it: every weight is used once, so the time is that of streaming
 // W from HBM, and a read-only stream only reaches the memory's rate if each
@@ -49,9 +50,10 @@ typedef __attribute__((__vector_size__(4 * sizeof(unsigned int)))) unsigned int
 
 enum End { ROWS, SILU, SUMS };
 
-// MT: 16-row tiles of x; RT: 8-row tiles of W per wave; NW: waves; KS: k per
-// slice; OCC: waves per SIMD that the registers have to allow
-template <int MT, int RT, int NW, int KS, int OCC, int END>
+// MT: 16-row tiles of x; RT: tiles of W per wave, of 8 rows as above or, with
+// HALF, of 16 rows read half a line at a time; NW: waves; KS: k per slice; OCC:
+// waves per SIMD that the registers have to allow
+template <int MT, int RT, int NW, int KS, int OCC, int END, bool HALF>
 __global__ __launch_bounds__(NW * WAVE, OCC) void stream_gemm_kernel(
     unsigned short* __restrict__ out,      // [M, N] bf16; SILU: [M, N / 2]
     float* __restrict__ sums,              // [splits, M, N] (SUMS)
@@ -60,6 +62,8 @@ __global__ __launch_bounds__(NW * WAVE, OCC) void stream_gemm_kernel(
     int M, int N, long K) {
   constexpr int NT = NW * WAVE;
   constexpr int ST = KS / 64;                  // steps per slice
+  constexpr int TR = HALF ? 16 : 8;            // rows of W per tile
+  constexpr int LW = HALF ? 2 : 1;             // loads per tile and step
   constexpr int XP = MT * 16 * KS / 8;         // 16-byte pieces of x per slice
   constexpr int XC = (XP + NT - 1) / NT;       // of them per thread
   __shared__ __align__(16) unsigned short xbuf[2][MT * 16 * KS];
@@ -70,15 +74,16 @@ __global__ __launch_bounds__(NW * WAVE, OCC) void stream_gemm_kernel(
 
   // with SILU the first half of a wave's tiles are gate rows, the others the
   // up rows of the same outputs
-  const int first = (blockIdx.x * NW + wid) * (END == SILU ? RT * 4 : RT * 8);
+  const int first =
+      (blockIdx.x * NW + wid) * (END == SILU ? RT * TR / 2 : RT * TR);
   const unsigned short* wp[RT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) {
-    const int tile_row = END != SILU ? first + i * 8
-                         : i < RT / 2 ? first + i * 8
-                                      : N / 2 + first + (i - RT / 2) * 8;
-    wp[i] = w + (long)(tile_row + (lane & 7)) * K +
-            (g + ((lane >> 3) & 1) * 4) * 8;
+    const int tile_row = END != SILU ? first + i * TR
+                         : i < RT / 2 ? first + i * TR
+                                      : N / 2 + first + (i - RT / 2) * TR;
+    wp[i] = w + (long)(tile_row + (lane & (TR - 1))) * K +
+            (HALF ? g : g + ((lane >> 3) & 1) * 4) * 8;
   }
 
   acc_t lo[RT][MT], hi[RT][MT];
@@ -109,15 +114,20 @@ __global__ __launch_bounds__(NW * WAVE, OCC) void stream_gemm_kernel(
           (((p % (KS / 8)) * 16) ^ ((row & 15) << 4))) = xr[i];
     }
   };
-  auto load_w = [&](int s, word4_t (&wv)[ST][RT]) {
+  auto load_w = [&](int s, word4_t (&wv)[ST][RT][LW]) {
 #pragma unroll
     for (int u = 0; u < ST; ++u)
 #pragma unroll
       for (int i = 0; i < RT; ++i)
-        wv[u][i] = __builtin_nontemporal_load(
-            reinterpret_cast<const word4_t*>(wp[i] + (long)s * KS + u * 64));
+#pragma unroll
+        for (int h = 0; h < LW; ++h) {
+          const auto* p = reinterpret_cast<const word4_t*>(
+              wp[i] + (long)s * KS + u * 64 + h * 32);
+          // half a line is better off kept for its other half
+          wv[u][i][h] = HALF ? *p : __builtin_nontemporal_load(p);
+        }
   };
-  auto multiply = [&](int b, const word4_t (&wv)[ST][RT]) {
+  auto multiply = [&](int b, const word4_t (&wv)[ST][RT][LW]) {
 #pragma unroll
     for (int u = 0; u < ST; ++u)
 #pragma unroll
@@ -130,17 +140,19 @@ __global__ __launch_bounds__(NW * WAVE, OCC) void stream_gemm_kernel(
             row + ((u * 128 + 64 + g * 16) ^ (c16 << 4)));
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
+          auto& other = HALF ? lo[i][m] : hi[i][m];
           lo[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(frag_t, wv[u][i]), x0, lo[i][m], 0, 0, 0);
-          hi[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(frag_t, wv[u][i]), x1, hi[i][m], 0, 0, 0);
+              __builtin_bit_cast(frag_t, wv[u][i][0]), x0, lo[i][m], 0, 0, 0);
+          other = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(frag_t, wv[u][i][LW - 1]), x1, other, 0, 0,
+              0);
         }
       }
   };
 
   const int step = gridDim.y;
   int s = blockIdx.y;
-  word4_t wa[ST][RT], wb[ST][RT];
+  word4_t wa[ST][RT][LW], wb[ST][RT][LW];
   load_x(s);
   load_w(s, wa);
   store_x(0);
@@ -162,8 +174,9 @@ __global__ __launch_bounds__(NW * WAVE, OCC) void stream_gemm_kernel(
     __syncthreads();
   }
 
-  // W row 4 * (g & 1) + r of tile i: lanes below 32 hold its first half
-  // lines' sum, lanes above its second half lines'
+  // With HALF a lane holds rows 4 * g + r of tile i. Otherwise W row
+  // 4 * (g & 1) + r: lanes below 32 hold its first half lines' sum, lanes above
+  // its second half lines'
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     float v[RT][4];
@@ -171,14 +184,14 @@ __global__ __launch_bounds__(NW * WAVE, OCC) void stream_gemm_kernel(
     for (int i = 0; i < RT; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        v[i][r] = g < 2 ? lo[i][m][r] : hi[i][m][r];
-        v[i][r] += __shfl_xor(v[i][r], 32, WAVE);
+        v[i][r] = HALF || g < 2 ? lo[i][m][r] : hi[i][m][r];
+        if (!HALF) v[i][r] += __shfl_xor(v[i][r], 32, WAVE);
       }
     const int row = m * 16 + c16;
-    if (g >= 2 || row >= M) continue;
+    if ((!HALF && g >= 2) || row >= M) continue;
 #pragma unroll
     for (int i = 0; i < (END == SILU ? RT / 2 : RT); ++i) {
-      const int n = first + i * 8 + g * 4;
+      const int n = first + i * TR + g * 4;
       if (END == SUMS) {
         *reinterpret_cast<float4*>(
             sums + ((long)blockIdx.y * M + row) * N + n) =
@@ -271,29 +284,43 @@ void launch(unsigned short* out, float* sums, int splits,
   const int M = x.size(0), N = w.size(0);
   const long K = x.size(1);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-#define SG_LAUNCH(MT_, RT_, KS_, OCC_)                                       \
-  stream_gemm_kernel<MT_, RT_, 8, KS_, OCC_, END>                            \
-      <<<dim3(N / (RT_ * 64), splits), 8 * WAVE, 0, stream>>>(               \
+#define SG_LAUNCH(MT_, RT_, KS_, OCC_, HALF_)                                \
+  stream_gemm_kernel<MT_, RT_, 8, KS_, OCC_, END, HALF_>                     \
+      <<<dim3(N / (RT_ * (HALF_ ? 128 : 64)), splits), 8 * WAVE, 0,          \
+         stream>>>(                                                          \
           out, sums, reinterpret_cast<const unsigned short*>(x.data_ptr()),  \
           reinterpret_cast<const unsigned short*>(w.data_ptr()), M, N, K)
   const int MT = (M + 15) / 16;
-  // Twice the rows per workgroup halve the passes of x through LDS, where that
-  // leaves most CUs one workgroup and none a second (57344 x 8192: M = 8 166 ->
-  // 156 us, 32 178 -> 159, 64 200 -> 183; but 128256 x 4096, M = 8 179 -> 203)
-  if (END != SUMS && N % 256 == 0 && N >= 200 * 256 && N <= 256 * 256) {
-    switch (MT) {
-      case 1: SG_LAUNCH(1, 4, 256, 2); break;
-      case 2: SG_LAUNCH(2, 4, 256, 2); break;
-      case 3: SG_LAUNCH(3, 4, 128, 2); break;
-      default: SG_LAUNCH(4, 4, 128, 2); break;
+  if constexpr (END == SUMS) {
+    // The matrix cores have nothing to spare any more: whole tiles of 16 rows
+    // (4096 x 14336: 33 us at M = 96, 35 at 128; hipBLASLt 65 and 76).
+    if (M > 64) {
+      if (M <= 96) { SG_LAUNCH(6, 1, 256, 2, true); }
+      else { SG_LAUNCH(8, 1, 256, 2, true); }
+      HIP_CHECK_KERNEL();
+      return;
     }
   } else {
-    switch (MT) {
-      case 1: SG_LAUNCH(1, 2, 256, 4); break;
-      case 2: SG_LAUNCH(2, 2, 256, 2); break;
-      case 3: SG_LAUNCH(3, 2, 256, 2); break;
-      default: SG_LAUNCH(4, 2, 256, 2); break;
+    // Twice the rows per workgroup halve the passes of x through LDS, where
+    // that leaves most CUs one workgroup and none a second (57344 x 8192: M = 8
+    // 166 -> 156 us, 32 178 -> 159, 64 200 -> 183; but 128256 x 4096, M = 8
+    // 179 -> 203)
+    if (N % 256 == 0 && N >= 200 * 256 && N <= 256 * 256) {
+      switch (MT) {
+        case 1: SG_LAUNCH(1, 4, 256, 2, false); break;
+        case 2: SG_LAUNCH(2, 4, 256, 2, false); break;
+        case 3: SG_LAUNCH(3, 4, 128, 2, false); break;
+        default: SG_LAUNCH(4, 4, 128, 2, false); break;
+      }
+      HIP_CHECK_KERNEL();
+      return;
     }
+  }
+  switch (MT) {
+    case 1: SG_LAUNCH(1, 2, 256, 4, false); break;
+    case 2: SG_LAUNCH(2, 2, 256, 2, false); break;
+    case 3: SG_LAUNCH(3, 2, 256, 2, false); break;
+    default: SG_LAUNCH(4, 2, 256, 2, false); break;
   }
 #undef SG_LAUNCH
   HIP_CHECK_KERNEL();
@@ -305,7 +332,7 @@ void check(const torch::Tensor& x, const torch::Tensor& w) {
   TORCH_CHECK(x.scalar_type() == torch::kBFloat16 &&
               w.scalar_type() == torch::kBFloat16);
   TORCH_CHECK(x.is_contiguous() && w.is_contiguous());
-  TORCH_CHECK(x.size(0) >= 1 && x.size(0) <= 64 && w.size(0) > 0 &&
+  TORCH_CHECK(x.size(0) >= 1 && x.size(0) <= 128 && w.size(0) > 0 &&
               w.size(0) % ROWS_PER_WG == 0 && x.size(1) > 0 &&
               x.size(1) % SLICE == 0);
   TORCH_CHECK(reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 &&
@@ -318,7 +345,7 @@ void check(const torch::Tensor& x, const torch::Tensor& w) {
 // 26.7, in 16 31.2).
 int splits_of(const torch::Tensor& x, const torch::Tensor& w) {
   const long rows = w.size(0) / ROWS_PER_WG;
-  if (rows >= 192) return 1;
+  if (rows >= 192 && x.size(0) <= 64) return 1;
   const long room = x.size(0) <= 16 ? 512 : 256;
   return (int)std::max(1L, std::min(room / rows, (long)x.size(1) / SLICE));
 }
@@ -345,7 +372,7 @@ unsigned short* bf16_rows(const torch::Tensor& t, long rows, long cols) {
 void stream_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
   check(x, w);
   auto* op = bf16_rows(out, x.size(0), w.size(0));
-  if (splits_of(x, w) == 1) {
+  if (x.size(0) <= 64 && splits_of(x, w) == 1) {
     launch<ROWS>(op, nullptr, 1, x, w);
     return;
   }
@@ -366,6 +393,7 @@ torch::Tensor stream_gemm_sums(torch::Tensor x, torch::Tensor w) {
 // out [M, N / 2] = silu(x W[:N/2]^T) * (x W[N/2:]^T)
 void stream_gemm_silu(torch::Tensor out, torch::Tensor x, torch::Tensor w) {
   check(x, w);
+  TORCH_CHECK(x.size(0) <= 64);
   launch<SILU>(bf16_rows(out, x.size(0), w.size(0) / 2), nullptr, 1, x, w);
 }
 
