@@ -339,14 +339,15 @@ void check(const torch::Tensor& x, const torch::Tensor& w) {
               reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0);
 }
 
-// Workgroups of the same rows that share their reduction: the chip holds 256
-// workgroups at a time, 512 of those that keep one tile of x (4096 x 14336, 32
-// workgroups of rows: M = 8 in 16 parts 20.4 us, in 8 21.5; M = 64 in 8 parts
-// 26.7, in 16 31.2).
+// Workgroups of the same rows that share their reduction: one for each of 256
+// CUs. The registers of one tile of x would let two share a CU, and the product
+// alone is then 1 us faster (4096 x 14336, M = 8: 20.4 us in 16 parts, 21.5 in
+// 8), but twice the parts cost who reads them more: with the norm 28.1 us and
+// 26.7, 8192 x 28672 96.8 and 86.2.
 int splits_of(const torch::Tensor& x, const torch::Tensor& w) {
   const long rows = w.size(0) / ROWS_PER_WG;
   if (rows >= 192 && x.size(0) <= 64) return 1;
-  const long room = x.size(0) <= 16 ? 512 : 256;
+  const long room = 256;
   return (int)std::max(1L, std::min(room / rows, (long)x.size(1) / SLICE));
 }
 
