@@ -563,13 +563,29 @@ def mlp_down_fused(gu: torch.Tensor, w: torch.Tensor,
     return linear_add_rmsnorm(act, w, residual, norm_weight, eps)
 
 
+def _mlp_stream_wins(rows: int, N: int, K: int) -> bool:
+    """Where the fused projection and activation beat hipBLASLt and silu_mul
+    (us, fused against the two, in a graph, weights from HBM). The activation
+    needs whole sums, so the rows of W alone fill the chip: with 28672 and more
+    of them always (28672 x 4096 44 to 62 at 8 rows, 51 to 56 at 64); with fewer
+    only while x is small (22016 x 4096 43 to 44 at 32 rows, 49 to 46 at 64;
+    14336 x 4096 29 to 32 at 16, 30 to 29 at 32; 8192 x 4096 23 to 19 at 8, but
+    8192 x 2048 13 to 17)."""
+    if N >= 24576:
+        return True
+    if rows <= 16:
+        return N >= 12288 or K <= 2048
+    return rows <= 32 and (N >= 20480 or K <= 2048)
+
+
 def mlp_act(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T) for the fused projection w = [Wg; Wu]. Decode
     batches do it in one kernel, with both factors in fp32; otherwise the
     projection is rounded to bf16 in between."""
     act = torch.empty(x.shape[0], w.shape[0] // 2, dtype=x.dtype,
                       device=x.device)
-    if w.shape[0] % 256 == 0 and _stream_ok(x, w):
+    if (w.shape[0] % 256 == 0 and _stream_ok(x, w)
+            and _mlp_stream_wins(x.shape[0], w.shape[0], w.shape[1])):
         _C.stream_gemm_silu(act, x, w)
     else:
         silu_mul(act, linear(x, w))

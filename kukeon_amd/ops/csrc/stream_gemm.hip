@@ -284,9 +284,9 @@ void launch(unsigned short* out, float* sums, int splits,
   const int M = x.size(0), N = w.size(0);
   const long K = x.size(1);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-#define SG_LAUNCH(MT_, RT_, KS_, OCC_, HALF_)                                \
-  stream_gemm_kernel<MT_, RT_, 8, KS_, OCC_, END, HALF_>                     \
-      <<<dim3(N / (RT_ * (HALF_ ? 128 : 64)), splits), 8 * WAVE, 0,          \
+#define SG_LAUNCH(MT_, RT_, NW_, KS_, OCC_, HALF_)                           \
+  stream_gemm_kernel<MT_, RT_, NW_, KS_, OCC_, END, HALF_>                   \
+      <<<dim3(N / (RT_ * NW_ * (HALF_ ? 16 : 8)), splits), NW_ * WAVE, 0,    \
          stream>>>(                                                          \
           out, sums, reinterpret_cast<const unsigned short*>(x.data_ptr()),  \
           reinterpret_cast<const unsigned short*>(w.data_ptr()), M, N, K)
@@ -295,32 +295,67 @@ void launch(unsigned short* out, float* sums, int splits,
     // The matrix cores have nothing to spare any more: whole tiles of 16 rows
     // (4096 x 14336: 33 us at M = 96, 35 at 128; hipBLASLt 65 and 76).
     if (M > 64) {
-      if (M <= 96) { SG_LAUNCH(6, 1, 256, 2, true); }
-      else { SG_LAUNCH(8, 1, 256, 2, true); }
+      if (M <= 96) { SG_LAUNCH(6, 1, 8, 256, 2, true); }
+      else { SG_LAUNCH(8, 1, 8, 256, 2, true); }
       HIP_CHECK_KERNEL();
       return;
     }
   } else {
+    // Without parts it is the rows that have to fill the chip: 7 waves to a
+    // workgroup where that makes more workgroups than 8 do and not more than
+    // there are CUs (28672 x 4096: 256 instead of 224).
+    const auto seven = [&](int rt) {
+      return N > 256 * 64 && N % (rt * 56) == 0 && N / (rt * 56) <= 256;
+    };
     // Twice the rows per workgroup halve the passes of x through LDS, where
     // that leaves most CUs one workgroup and none a second (57344 x 8192: M = 8
     // 166 -> 156 us, 32 178 -> 159, 64 200 -> 183; but 128256 x 4096, M = 8
     // 179 -> 203)
-    if (N % 256 == 0 && N >= 200 * 256 && N <= 256 * 256) {
+    const bool wide = N % 256 == 0 && N >= 200 * 256 && N <= 256 * 256;
+#define SG_WIDE(NW_)                                                         \
+  switch (MT) {                                                              \
+    case 1: SG_LAUNCH(1, 4, NW_, 256, 2, false); break;                      \
+    case 2: SG_LAUNCH(2, 4, NW_, 256, 2, false); break;                      \
+    case 3: SG_LAUNCH(3, 4, NW_, 128, 2, false); break;                      \
+    default: SG_LAUNCH(4, 4, NW_, 128, 2, false); break;                     \
+  }
+    if (wide || seven(2)) {
+      if (wide && seven(4)) {
+        SG_WIDE(7)
+      } else if (wide) {
+        SG_WIDE(8)
+      } else {
+        switch (MT) {
+          case 1: SG_LAUNCH(1, 2, 7, 256, 4, false); break;
+          case 2: SG_LAUNCH(2, 2, 7, 256, 2, false); break;
+          case 3: SG_LAUNCH(3, 2, 7, 256, 2, false); break;
+          default: SG_LAUNCH(4, 2, 7, 256, 2, false); break;
+        }
+      }
+      HIP_CHECK_KERNEL();
+      return;
+    }
+#undef SG_WIDE
+  }
+  if constexpr (END == SILU) {
+    // the activation cannot be split into parts: few rows take half as many
+    // waves to a workgroup
+    if (N <= 256 * 64) {
       switch (MT) {
-        case 1: SG_LAUNCH(1, 4, 256, 2, false); break;
-        case 2: SG_LAUNCH(2, 4, 256, 2, false); break;
-        case 3: SG_LAUNCH(3, 4, 128, 2, false); break;
-        default: SG_LAUNCH(4, 4, 128, 2, false); break;
+        case 1: SG_LAUNCH(1, 2, 4, 256, 2, false); break;
+        case 2: SG_LAUNCH(2, 2, 4, 256, 2, false); break;
+        case 3: SG_LAUNCH(3, 2, 4, 256, 2, false); break;
+        default: SG_LAUNCH(4, 2, 4, 256, 2, false); break;
       }
       HIP_CHECK_KERNEL();
       return;
     }
   }
   switch (MT) {
-    case 1: SG_LAUNCH(1, 2, 256, 4, false); break;
-    case 2: SG_LAUNCH(2, 2, 256, 2, false); break;
-    case 3: SG_LAUNCH(3, 2, 256, 2, false); break;
-    default: SG_LAUNCH(4, 2, 256, 2, false); break;
+    case 1: SG_LAUNCH(1, 2, 8, 256, 4, false); break;
+    case 2: SG_LAUNCH(2, 2, 8, 256, 2, false); break;
+    case 3: SG_LAUNCH(3, 2, 8, 256, 2, false); break;
+    default: SG_LAUNCH(4, 2, 8, 256, 2, false); break;
   }
 #undef SG_LAUNCH
   HIP_CHECK_KERNEL();

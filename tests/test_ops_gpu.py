@@ -958,7 +958,8 @@ def _close(got, want, scale):
 # row tiles of x (16), units of W (128 rows, 256 columns), one part and many
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 33, 49, 64, 65, 97, 128])
 @pytest.mark.parametrize("N,K", [(128, 256), (256, 768), (2048, 4096),
-                                 (24576, 512), (51200, 256)])
+                                 (24576, 512), (51200, 256), (17920, 256),
+                                 (57344, 256)])
 def test_stream_gemm(M, N, K):
     torch.manual_seed(M + N)
     x = torch.randn(M, K, dtype=torch.bfloat16, device=DEV)
