@@ -21,6 +21,8 @@
 //  [6..7] packed argmax (u64, 8-byte aligned: 528*4 % 8 == 0)
 //  [8]  need_k (f32)          [9] need_p (f32)
 //  [16..271] hist_count (u32) [272..527] hist_weight (f32)
+#include <algorithm>
+
 #include "common.h"
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
@@ -373,16 +375,19 @@ __global__ void decode_advance_kernel(int* __restrict__ ids,
                                       const int* __restrict__ tokens,
                                       int* __restrict__ ring,
                                       int* __restrict__ counter, int B) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
   const int step = counter[0];
-  if (seq_lens[b] > 0) {  // active rows only (padded rows stay parked)
-    ids[b] = tokens[b];
-    pos[b] += 1;
-    seq_lens[b] += 1;
-    ring[step * B + b] = tokens[b];
+  // all waves have the step before one of them moves it on: a wave that came
+  // late wrote its tokens to the next step's line (more than 64 rows)
+  __syncthreads();
+  for (int b = threadIdx.x; b < B; b += blockDim.x) {
+    if (seq_lens[b] > 0) {  // active rows only (padded rows stay parked)
+      ids[b] = tokens[b];
+      pos[b] += 1;
+      seq_lens[b] += 1;
+      ring[step * B + b] = tokens[b];
+    }
   }
-  if (b == 0) counter[0] = step + 1;
+  if (threadIdx.x == 0) counter[0] = step + 1;
 }
 
 void decode_advance(torch::Tensor ids, torch::Tensor pos,
@@ -390,7 +395,9 @@ void decode_advance(torch::Tensor ids, torch::Tensor pos,
                     torch::Tensor ring, torch::Tensor counter) {
   const int B = ids.size(0);
   auto stream = c10::hip::getCurrentHIPStream().stream();
-  decode_advance_kernel<<<(B + 255) / 256, 256, 0, stream>>>(
+  // one workgroup: the step counter is read and moved on within it
+  decode_advance_kernel<<<1, std::max(64, std::min(1024, (B + 63) / 64 * 64)),
+                          0, stream>>>(
       ids.data_ptr<int>(), pos.data_ptr<int>(), seq_lens.data_ptr<int>(),
       tokens.data_ptr<int>(), ring.data_ptr<int>(), counter.data_ptr<int>(),
       B);

@@ -1102,3 +1102,25 @@ def test_paged_attention_pieces(Hq, Hk, splits, lens, fp8):
     tol = 7e-2 if fp8 else 2.5e-2
     torch.testing.assert_close(out.cpu().float(), ref.float(), rtol=tol,
                                atol=tol)
+
+
+# rows of one wave, of several, and more than a workgroup's threads
+@pytest.mark.parametrize("B", [1, 64, 65, 256, 300, 1500])
+def test_decode_advance_steps(B):
+    """Every row's token of a step is in that step's line of the ring."""
+    steps = 50
+    lens = torch.arange(B, dtype=torch.int32, device=DEV) % 5
+    live = lens > 0
+    ids, pos = torch.zeros_like(lens), lens.clone()
+    ring = torch.full((steps * B,), -1, dtype=torch.int32, device=DEV)
+    counter = torch.zeros(1, dtype=torch.int32, device=DEV)
+    seq = lens.clone()
+    made = torch.randint(0, 1 << 20, (steps, B), dtype=torch.int32,
+                         device=DEV)
+    for t in range(steps):
+        ops.decode_advance(ids, pos, seq, made[t], ring, counter)
+    want = torch.where(live, made, -1)
+    assert torch.equal(ring.view(steps, B), want)
+    assert torch.equal(ids, torch.where(live, made[-1], 0))
+    assert torch.equal(seq, torch.where(live, lens + steps, lens))
+    assert torch.equal(pos, seq) and counter.item() == steps
