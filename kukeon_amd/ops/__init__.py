@@ -315,12 +315,11 @@ _SKINNY_WS = {}
 # captured earlier may still hold the old tensor's device pointer, and
 # letting it free would put a use-after-free inside every later replay
 _SKINNY_WS_RETIRED = []
-# Per-shape dispatch, from the measured sweep (profiles/r01_progress.md,
-# scripts/sweep_splitk.py on MI355X): the glds-staged skinny kernel beats
-# hipBLASLt on square o-projection shapes (N==K: 16.6us vs 19.3 at M=64,
-# 11.9 vs 19.2 at M=16 on 4096x4096) and trails it on qkv/gate_up/down/
-# lm_head, where hipBLASLt is 55-100% of the HBM floor. KUKEON_SKINNY_GEMM=1
-# forces the skinny kernel for every eligible shape (benchmarking).
+# The skinny kernels serve what _stream_ok leaves (autocast, reductions that are
+# no multiple of 256) and, with KUKEON_SKINNY_GEMM=1 or 5, every eligible shape.
+# The first of them beats hipBLASLt on square output projections (N==K: 16.6us
+# vs 19.3 at M=64, 11.9 vs 19.2 at M=16 on 4096x4096) and trails it on qkv,
+# gate_up, down and the head; the streaming kernel takes 8 and 11 there.
 _USE_SKINNY = __import__("os").environ.get("KUKEON_SKINNY_GEMM", "0")
 # silu-into-down-staging fusion: measured SLOWER in situ (54.2us fused vs
 # 42.9 for silu_mul + gemm cold; bench 51.7 vs 53.6 turns/s same box) —
@@ -366,7 +365,9 @@ def _stream_ok(x: torch.Tensor, w: torch.Tensor, most: int = 64) -> bool:
             and w.shape[0] % 128 == 0 and w.shape[1] % 256 == 0
             and w.numel() >= 1 << 21
             and x.is_contiguous() and w.is_contiguous()
-            # what records, batches or traces goes through torch
+            # the kernels take the current device's stream
+            and x.device.index == torch.cuda.current_device()
+            # what records, batches, traces or casts goes through torch
             and type(x) is torch.Tensor
             and type(w) in (torch.Tensor, torch.nn.Parameter)
             and not (torch.is_grad_enabled()
@@ -374,6 +375,8 @@ def _stream_ok(x: torch.Tensor, w: torch.Tensor, most: int = 64) -> bool:
             and not torch._C._are_functorch_transforms_active()
             and torch.autograd.forward_ad._current_level < 0
             and not torch.jit.is_tracing()
+            and not torch.is_autocast_enabled("cuda")
+            and torch._C._len_torch_dispatch_stack() == 0
             and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
@@ -476,7 +479,10 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor,
     rows = x.shape[0]
     N, K = w.shape
     if (parallel.tp_size() == 1 and N % 2048 == 0 and N <= 8192
-            and residual.is_contiguous() and _stream_ok(x, w, 128)):
+            and _stream_ok(x, w, 128)
+            and all(t.dtype == torch.bfloat16 and t.device == x.device
+                    and t.is_contiguous() and t.data_ptr() % 8 == 0
+                    for t in (residual, norm_weight))):
         normed = torch.empty(rows, N, dtype=x.dtype, device=x.device)
         _C.stream_gemm_norm(normed, x, w, residual, norm_weight, eps)
         return normed

@@ -1058,6 +1058,9 @@ def test_stream_dispatch():
         assert not ops._stream_ok(xx, ww)
         torch.testing.assert_close(ops.linear(xx, ww),
                                    torch.nn.functional.linear(xx, ww))
+    with torch.autocast("cuda", torch.float16):
+        assert not ops._stream_ok(x, w)
+        assert ops.linear(x[:16], w).dtype == torch.float16
     y = torch.vmap(lambda r: ops.linear(r, w))(x.view(4, 16, 2048))
     torch.testing.assert_close(y.view(64, -1).float(),
                                torch.nn.functional.linear(x, w).float(),
