@@ -5,8 +5,7 @@
 // normalize pass so each row is read from HBM exactly once.
 //
 // Capability parity note: the reference (eminwux/kukeon) has no GPU ops; this
-// is part of the new data plane required by BASELINE.json (hand-written CDNA4
-// RMSNorm kernel).
+// is part of the data plane.
 #include "common.h"
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>

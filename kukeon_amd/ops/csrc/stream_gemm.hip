@@ -23,7 +23,7 @@
 //   - matrices of few rows split the reduction over workgroups until the chip
 //     is full; whoever reads the result next adds the partial sums up.
 // Measured, M = 8 / 32 / 64, weights from HBM, in us (hipBLASLt beside it):
-//   28672 x 4096   42 / 46 / 50   (62 / 51 / 52)
+//   28672 x 4096   44 / 45 / 52   (62 / 51 / 52), with the activation
 //   4096 x 14336   20 / 22 / 27   (28 / 32 / 40)
 //   6144 x 4096    11 / 13 / 16   (21 / 19 / 19)
 //   4096 x 4096     8 /  9 / 11   (21 / 19 / 19)
@@ -303,7 +303,8 @@ void launch(unsigned short* out, float* sums, int splits,
   } else {
     // Without parts it is the rows that have to fill the chip: 7 waves to a
     // workgroup where that makes more workgroups than 8 do and not more than
-    // there are CUs (28672 x 4096: 256 instead of 224).
+    // there are CUs (28672 x 4096: 256 instead of 224, with the activation 44.4
+    // -> 43.5 us at 8 rows and 48.3 -> 45.2 at 32; 57344 x 8192 167.8 -> 159.8).
     const auto seven = [&](int rt) {
       return N > 256 * 64 && N % (rt * 56) == 0 && N / (rt * 56) <= 256;
     };
@@ -339,7 +340,7 @@ void launch(unsigned short* out, float* sums, int splits,
   }
   if constexpr (END == SILU) {
     // the activation cannot be split into parts: few rows take half as many
-    // waves to a workgroup
+    // waves to a workgroup (14336 x 4096, 8 rows: 38.4 -> 28.5 us)
     if (N <= 256 * 64) {
       switch (MT) {
         case 1: SG_LAUNCH(1, 2, 4, 256, 2, false); break;
